@@ -90,19 +90,30 @@ __device__ __forceinline__ float expf_fast(float x) { return __builtin_amdgcn_ex
 // opacity >= 1/255: <= ~5e-7) plus the cut-off's own rounding (~1e-6).
 constexpr float ALPHA_GUARD = 3e-5f;
 
-// alpha = min(0.99, opacity * G) of one (pixel, Gaussian) evaluation with the
-// fast exp; where power lies within ALPHA_GUARD of the Gaussian's cut-off
-// power (any lane of the wave), G is the exact expf_nonpos instead, so the
-// decision alpha >= 1/255 is the one the exact evaluation makes.  The window
-// test needs only power, not the exp, so the exp's latency overlaps it.  G is
-// returned too.
-__device__ __forceinline__ float blend_alpha(float opacity, float power, float cut_power, float& G)
+// G of one (pixel, Gaussian) evaluation with the fast exp; where power lies
+// within ALPHA_GUARD of the Gaussian's cut-off power (any lane of the wave), G
+// is the exact expf_nonpos instead, so the decision alpha >= 1/255 is the one
+// the exact evaluation makes.  The window test needs only power, not the exp,
+// so the exp's latency overlaps it.
+__device__ __forceinline__ float blend_g(float power, float cut_power)
 {
     const bool near = __builtin_fabsf(power - cut_power) <= ALPHA_GUARD;
-    G = expf_fast(power);
+    float G = expf_fast(power);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(near) != 0, 0)) {
         if (near) G = expf_nonpos(power);
     }
+    return G;
+}
+
+__device__ __forceinline__ float blend_opacity_g(float opacity, float power, float cut_power)
+{
+    return opacity * blend_g(power, cut_power);
+}
+
+// alpha = min(0.99, opacity * G); G is returned too
+__device__ __forceinline__ float blend_alpha(float opacity, float power, float cut_power, float& G)
+{
+    G = blend_g(power, cut_power);
     return __builtin_fminf(0.99f, opacity * G);
 }
 

@@ -3174,20 +3174,14 @@ __global__ __launch_bounds__(256) void unpack_map_grads_kernel(int P, const int*
         g_map[(size_t)NUM_MAPS * i + c] = cx >= 0 ? gacc[(size_t)cx * 16 + 11 + c] : 0.f;
 }
 
-// Per-pixel state and constants of the backward blend, and the backward of
-// one staged entry for one pixel: updates the state and returns whether the
-// pixel blends the entry, with its eleven gradient terms in vals (dmean x, y,
-// |dmean x|, |dmean y|, dconic a, b, c, dopacity, drgb; vals[11] = 0).
-// Shared by the backward kernels and the VALU probe (render_valu_probe).
-// Per-pixel state of the backward walk.  The accumulated colour behind the
-// current entry and the last blended colour enter the gradient only through
-// their dot products with dL/dpixel, and the accumulation is linear, so the
-// state keeps those two dot products instead of the six channel values.
+// Per-pixel state of the backward walk (shared, like bwd_eval and bwd_apply,
+// by the backward kernels and the VALU probe).  The accumulated colour behind
+// the current entry enters the gradient only through its dot product with
+// dL/dpixel, and the accumulation is linear, so the state keeps that dot
+// product instead of the three channel values.
 struct BwdPixel {
-    float T;            // transmittance in front of the current entry
-    float acc_dp;       // (colour accumulated behind it) . dL/dpixel
-    float last_dp;      // (colour of the last blended entry) . dL/dpixel
-    float last_alpha;
+    float T;        // transmittance in front of the current entry
+    float acc_dp;   // (colour accumulated behind it) . dL/dpixel
 };
 
 struct BwdConst {
@@ -3199,9 +3193,10 @@ struct BwdConst {
 // decides whether the pixel blends the entry (the forward's exact alpha
 // expressions), and bwd_apply, which the caller skips when no lane of the
 // wave blends it (the state update is then the identity for every lane),
-// updates the pixel's state and yields the entry's twelve gradient terms.
+// updates the pixel's state and yields the entry's gradient factors.
 struct BwdEval {
-    float dx, dy, hadx, hcdy, nbdx, alpha, G0;
+    float dy, hadx, hcdy, nbdx;
+    float oG;   // opacity G, 0 where the pixel does not blend the entry
     bool valid;
 };
 
@@ -3209,81 +3204,259 @@ __device__ __forceinline__ BwdEval bwd_eval(const BwdConst& k, const float4& A, 
 {
     BwdEval e;
     const int ci1 = __float_as_int(Cc.z);   // 1-based position in the tile's list
-    e.dx = A.x - k.pxf;
+    const float dx = A.x - k.pxf;
     e.dy = A.y - k.pyf;
     // gs::power_of's operations, with the products ha dx, hc dy, nb dx kept
     // for the gradient
-    e.hadx = A.z * e.dx;
+    e.hadx = A.z * dx;
     e.hcdy = B.x * e.dy;
-    e.nbdx = A.w * e.dx;
-    const float power = __builtin_fmaf(e.hadx, e.dx, __builtin_fmaf(e.hcdy, e.dy, e.nbdx * e.dy));
-    e.alpha = gs::blend_alpha(B.y, power, Cc.w, e.G0);
-    e.valid = ci1 <= k.last && !(power > 0.0f) && !(e.alpha < (1.0f / 255.0f));
+    e.nbdx = A.w * dx;
+    const float power = __builtin_fmaf(e.hadx, dx, __builtin_fmaf(e.hcdy, e.dy, e.nbdx * e.dy));
+    // alpha = min(0.99, opacity G): its cut at 1/255 is opacity G's
+    const float oG = gs::blend_opacity_g(B.y, power, Cc.w);
+    e.valid = ci1 <= k.last && !(power > 0.0f) && !(oG < (1.0f / 255.0f));
+    e.oG = e.valid ? oG : 0.f;
     return e;
 }
 
+// a summed over lanes l and l ^ 32 in the lanes < 32, b in the others
+__device__ __forceinline__ float swap32_add(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// the same over lanes l and l ^ 16: a in the lanes with bit 4 clear
+__device__ __forceinline__ float swap16_add(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// An entry's per-pixel gradient factors.  With w = dL/dG G, v = alpha T and
+// d = mean - pixel, every gradient term of the entry is a sum over the pixels
+// of w or v times a per-pixel constant, of |w dG/dmean| or (FULL) of the
+// unclamped w:  dmean = sum w (2 ha dx + nb dy, 2 hc dy + nb dx), dconic ~
+// sum w (dx dx, dx dy, dy dy), dopacity = sum w / opacity, drgb = sum v dL/dpixel.
+struct BwdTerms {
+    float w, v;
+    float u;   // split: |w dpx| (lanes < 32) and |w dpy| (>= 32), each summed over lanes l and l ^ 32;
+               // FULL: w where the alpha clamp is active too
+};
+
 // Branch-free: every lane applies the entry; a lane whose pixel does not
 // blend it (past its last contributor, power > 0, alpha < 1/255) gets zero
-// gradient factors and unchanged state, through selects on three factors
-// instead of per-value zeroing.  GEO (render_geo): m_dp is the entry's five
+// gradient factors and unchanged state through the one factor opacity G.  GEO (render_geo): m_dp is the entry's five
 // maps dotted with the pixel's map gradients; the maps join the colour in
 // every dot product (the accumulation is the same linear rule for all eight
-// channels).  Returns alpha T, the factor of the colour and map gradients.
+// channels).
 template <bool FULL, bool GEO = false>
-__device__ __forceinline__ float bwd_apply(BwdPixel& p, const BwdConst& k, const float4& A, const float4& B,
-                                           const float4& Cc, const BwdEval& e, float (&vals)[12],
-                                           [[maybe_unused]] float m_dp = 0.f)
+__device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, const float4& A, const float4& B,
+                                              const float4& Cc, const BwdEval& e,
+                                              [[maybe_unused]] float m_dp = 0.f)
 {
-    const bool valid = e.valid;
-    const float dx = e.dx, dy = e.dy;
-    // a lane that does not blend the entry runs it with alpha = 0 and G = 0:
-    // T is unchanged (1 / (1 - 0) is exactly 1), and every gradient term
-    // carries a factor alpha (colour) or G (the others; dL/dalpha stays finite)
-    const float alpha = valid ? e.alpha : 0.f;
-    const float G = valid ? e.G0 : 0.f;
+    // a lane that does not blend the entry runs it with opacity G = alpha = 0:
+    // T and the colour behind it are unchanged (1 / (1 - 0) is exactly 1), and
+    // every gradient term carries a factor alpha (colour) or opacity G (the
+    // others; dL/dalpha stays finite)
+    const float alpha = __builtin_fminf(0.99f, e.oG);
     const float inv_one_m = __builtin_amdgcn_rcpf(1.f - alpha);   // 1 ulp; gradients only
     p.T = p.T * inv_one_m;
-    const float dchannel_dcolor = alpha * p.T;
+    BwdTerms t;
+    t.v = alpha * p.T;
     // the reference's expressions, regrouped into fused multiply-adds and
     // taken in their dot products with dL/dpixel (gradients carry a
     // tolerance, not bit-exactness):
-    //   acc = la * lc + (1 - la) * acc        -> acc.dp += la * (lc.dp - acc.dp)
     //   dL/dalpha = sum_ch (c - acc) dp_ch    -> c.dp - acc.dp
-    //   (ha = -a/2, nb = -b, hc = -c/2 are the staged conic terms);
-    // a lane that does not blend the entry updates acc with factor 0
-    const float la = valid ? p.last_alpha : 0.f;
-    p.acc_dp = __builtin_fmaf(la, p.last_dp - p.acc_dp, p.acc_dp);
+    //   acc' = alpha c + (1 - alpha) acc      -> acc.dp += alpha (c.dp - acc.dp)
+    //   (ha = -a/2, nb = -b, hc = -c/2 are the staged conic terms)
     float c_dp = __builtin_fmaf(B.z, k.dp0, __builtin_fmaf(B.w, k.dp1, Cc.x * k.dp2));
     if constexpr (GEO) c_dp += m_dp;
-    p.last_dp = valid ? c_dp : p.last_dp;
-    p.last_alpha = valid ? alpha : p.last_alpha;
-    float dL_dalpha = c_dp - p.acc_dp;
-    const float gc0 = dchannel_dcolor * k.dp0;
-    const float gc1 = dchannel_dcolor * k.dp1;
-    const float gc2 = dchannel_dcolor * k.dp2;
-    dL_dalpha = __builtin_fmaf(dL_dalpha, p.T, inv_one_m * k.nT_bg);
-    const float dL_dG = B.y * dL_dalpha;
-    // dG/ddelx = G (2 ha dx + nb dy), dG/ddely = G (2 hc dy + nb dx)
-    const float dpx = __builtin_fmaf(2.0f, e.hadx, A.w * dy);
-    const float dpy = __builtin_fmaf(2.0f, e.hcdy, e.nbdx);
-    const float wG = dL_dG * G;
-    // the constant factors dmean/dpixel (W/2, H/2) and the conic terms' -1/2
-    // are applied once to the sums (unpack_grads_kernel), not per entry
-    const float gmx = wG * dpx;
-    const float gmy = wG * dpy;
-    const float wdx = wG * dx;
-    const bool clamped = FULL && B.y * G > 0.99f;
-    const float gca = clamped ? 0.f : wdx * dx;
-    const float gcb = clamped ? 0.f : wdx * dy;
-    const float gcc = clamped ? 0.f : (wG * dy) * dy;
-    const float gop = clamped ? 0.f : G * dL_dalpha;
-    // vals[2], vals[3]: |dmean| terms, made absolute by wave_sum12<true>
-    vals[0] = gmx; vals[1] = gmy; vals[2] = gmx; vals[3] = gmy;
-    vals[4] = gca; vals[5] = gcb; vals[6] = gcc; vals[7] = gop;
-    // slot 11 is never read back: any register that is dead here fills it
-    // (no zero has to be materialised for it)
-    vals[8] = gc0; vals[9] = gc1; vals[10] = gc2; vals[11] = dx;
-    return dchannel_dcolor;
+    const float d_dp = e.valid ? c_dp - p.acc_dp : 0.f;   // (a colour that is not finite stays with the pixels it enters)
+    p.acc_dp = __builtin_fmaf(alpha, d_dp, p.acc_dp);
+    const float dL_dalpha = __builtin_fmaf(d_dp, p.T, inv_one_m * k.nT_bg);
+    const float w = dL_dalpha * e.oG;
+    if constexpr (FULL) {
+        t.w = e.oG > 0.99f ? 0.f : w;
+        t.u = w;
+    } else {
+        // dG/ddelx = G (2 ha dx + nb dy), dG/ddely = G (2 hc dy + nb dx)
+        const float dpx = __builtin_fmaf(2.0f, e.hadx, A.w * e.dy);
+        const float dpy = __builtin_fmaf(2.0f, e.hcdy, e.nbdx);
+        t.w = w;
+        t.u = swap32_add(__builtin_fabsf(w) * __builtin_fabsf(dpx), __builtin_fabsf(w) * __builtin_fabsf(dpy));
+    }
+    return t;
+}
+
+// ---- the wave's gradient sums, four entries at a time.
+//
+// Each blended entry leaves its rows w, v, u (64 pixels) in LDS; after four,
+// lane l takes entry (l >> 1) & 3 and four consecutive pixels of it, forms
+// the entry's eleven terms summed over those four (the w moments from sum w,
+// sum i w, sum i i w) and the terms are summed over the entry's sixteen lanes.
+//
+// Bound: the walk is bound by VALU issue.  Forming the eleven terms per pixel
+// and summing each over 64 lanes by transpose-adds took 36 VALU instructions
+// of an entry's 84; this takes 19 (and 5 for the rows).  Measured (render
+// backward, before -> after): 6M aerial Gaussians at 1600x1066 642 -> 510 us,
+// 1M wide ones at 1920x1080 367 -> 284 us, the full-image path's 2M at
+// 1237x822 377 -> 225 us.  Tried: the sums as a contraction on the matrix
+// cores, v_mfma_f32_16x16x4_f32 with four entries' rows against per-pixel
+// constants (equal accuracy): 700 us at 6M, because a float32 MFMA and the
+// VALU do not overlap on this target (a loop of one MFMA and 16 FMAs takes 108
+// cycles, of either alone 34 and 71; a bf16 MFMA does overlap, but splitting
+// the rows into three bf16 parts costs more VALU than it saves); eight entries
+// of eight pixels per lane (fewer instructions, but four waves per SIMD and
+// twice the accumulator lines per entry): 508 -> 594 us at 6M.
+constexpr int GRAD_SLOTS = 4;          // entries per flush
+constexpr int GRAD_STRIDE = 3 * 64 + 8;   // floats per slot: 3 rows, and 8 more so that 8 lanes' 16-byte reads meet 32 banks
+
+// orders this wave's LDS accesses (one wave per block: they execute in order)
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the four pixels of a lane: their number in the quadrant is 4 q .. 4 q + 3
+__device__ __forceinline__ int grad_chunk(int lane) { return (lane >> 3) * 2 + (lane & 1); }
+
+template <bool GEO>
+struct GradPixels {
+    float dp[3][4];                  // dL/dpixel of the lane's four pixels
+    float dm[GEO ? NUM_MAPS : 1][4]; // render_geo: their map gradients
+    float x0, y;                     // the first one's position
+};
+
+// every lane's pixel constants, redistributed through LDS (rows: NUM_MAPS + 3
+// rows of 64 fit)
+template <bool GEO>
+__device__ __forceinline__ GradPixels<GEO> grad_pixels(float* rows, int lane, float qx0, float qy0, float dp0,
+                                                       float dp1, float dp2, const float (&dm)[NUM_MAPS])
+{
+    static_assert(GRAD_SLOTS * GRAD_STRIDE >= (NUM_MAPS + 3) * 64, "rows too small");
+    rows[lane] = dp0;
+    rows[64 + lane] = dp1;
+    rows[128 + lane] = dp2;
+    if constexpr (GEO) {
+        for (int c = 0; c < NUM_MAPS; c++) rows[(3 + c) * 64 + lane] = dm[c];
+    }
+    lds_order();
+    GradPixels<GEO> g;
+    const int q = grad_chunk(lane);
+    auto take = [&](int row, float (&o)[4]) {
+        const float4 v = *reinterpret_cast<const float4*>(rows + row * 64 + 4 * q);
+        o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+    };
+    for (int c = 0; c < 3; c++) take(c, g.dp[c]);
+    if constexpr (GEO) {
+        for (int c = 0; c < NUM_MAPS; c++) take(3 + c, g.dm[c]);
+    }
+    g.x0 = qx0 + (float)(4 * (q & 1));
+    g.y = qy0 + (float)(q >> 1);
+    lds_order();
+    return g;
+}
+
+__device__ __forceinline__ void grad_put(float* rows, int slot, int lane, const BwdTerms& t)
+{
+    float* r = rows + slot * GRAD_STRIDE + lane;
+    r[0] = t.w;
+    r[64] = t.v;
+    r[128] = t.u;
+}
+
+// Sums over the sixteen lanes of each entry (lanes that differ in bits 5, 4,
+// 3 and 0), as transpose-adds: the value of accumulator slot i = (bit 5) + 2
+// (bit 4) + 4 (bit 3) + 8 (bit 0) ends in the lane with those bits.  p01 ..
+// hold slots 0 and 1, ... (summed over bit 5 already).
+template <bool GEO>
+__device__ __forceinline__ float grad_reduce(float p01, float p23, float p45, float p67, float p89, float pab,
+                                             float pcd, float pef, int lane)
+{
+    const float t0 = swap16_add(p01, p23), t1 = swap16_add(p45, p67), t2 = swap16_add(p89, pab);
+    const bool lo8 = (lane & 8) == 0, even = (lane & 1) == 0;
+    const float z0 = (lo8 ? t0 : t1) + gs::dpp_f<0x128>(lo8 ? t1 : t0);   // row_ror:8
+    float z1;
+    if constexpr (GEO) {
+        const float t3 = swap16_add(pcd, pef);
+        z1 = (lo8 ? t2 : t3) + gs::dpp_f<0x128>(lo8 ? t3 : t2);
+    } else {
+        z1 = t2 + gs::dpp_f<0x128>(t2);
+    }
+    return (even ? z0 : z1) + gs::dpp_f<0xb1>(even ? z1 : z0);            // quad_perm [1,0,3,2]
+}
+
+__device__ __forceinline__ int grad_slot(int lane)
+{
+    return (lane >> 5) + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1) * 4 + (lane & 1) * 8;
+}
+
+struct GradSum {
+    float v;       // the term of accumulator slot grad_slot(lane)
+    uint32_t cx;   // of this accumulator row
+};
+
+// The sums of the slots' entries; byte e of `slots` is the staged position of
+// slot e's entry.  grad_flush adds the first n slots' to the accumulators.
+template <bool FULL, bool GEO>
+__device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels<GEO>& g, const Stage& st,
+                                             uint32_t slots, int lane)
+{
+    lds_order();
+    const int e = (lane >> 1) & 3;
+    const float* r = rows + e * GRAD_STRIDE + 4 * grad_chunk(lane);
+    const float4 w = *reinterpret_cast<const float4*>(r);
+    const float4 v = *reinterpret_cast<const float4*>(r + 64);
+    const float4 u = *reinterpret_cast<const float4*>(r + 128);
+    const int j = (int)((slots >> (8 * e)) & 63u);
+    const float4 A = st.a[j];
+    const float2 B = *reinterpret_cast<const float2*>(&st.b[j]);
+    const uint32_t cx = __float_as_uint(st.c[j].y);
+    const float dx = A.x - g.x0, dy = A.y - g.y;   // the first pixel's; the others' dx - 1, - 2, - 3
+    const float s = (w.x + w.y) + (w.z + w.w);
+    const float i1 = __builtin_fmaf(3.f, w.w, __builtin_fmaf(2.f, w.z, w.y));
+    const float i2 = __builtin_fmaf(9.f, w.w, __builtin_fmaf(4.f, w.z, w.y));
+    const float wx = __builtin_fmaf(dx, s, -i1), wy = dy * s;
+    const float wxx = __builtin_fmaf(dx, wx, __builtin_fmaf(-dx, i1, i2)), wxy = dy * wx, wyy = dy * wy;
+    float fx = wx, fy = wy, p23;
+    if constexpr (FULL) {
+        const float f = (u.x + u.y) + (u.z + u.w);
+        fx = __builtin_fmaf(dx, f, -__builtin_fmaf(3.f, u.w, __builtin_fmaf(2.f, u.z, u.y)));
+        fy = dy * f;
+        p23 = 0.f;   // not read
+    } else {
+        p23 = (u.x + u.y) + (u.z + u.w);
+    }
+    const float gx = __builtin_fmaf(2.f * A.z, fx, A.w * fy), gy = __builtin_fmaf(2.f * B.x, fy, A.w * fx);
+    const float gop = s * __builtin_amdgcn_rcpf(B.y);
+    auto dot = [&](const float (&d)[4]) {
+        return __builtin_fmaf(v.w, d[3], __builtin_fmaf(v.z, d[2], __builtin_fmaf(v.y, d[1], v.x * d[0])));
+    };
+    const float c2 = dot(g.dp[2]);
+    float pab, pcd = 0.f, pef = 0.f;
+    if constexpr (GEO) {
+        pab = swap32_add(c2, dot(g.dm[0]));
+        pcd = swap32_add(dot(g.dm[1]), dot(g.dm[2]));
+        pef = swap32_add(dot(g.dm[3]), dot(g.dm[4]));
+    } else {
+        pab = swap32_add(c2, c2);
+    }
+    const float sum = grad_reduce<GEO>(swap32_add(gx, gy), p23, swap32_add(wxx, wxy), swap32_add(wyy, gop),
+                                       swap32_add(dot(g.dp[0]), dot(g.dp[1])), pab, pcd, pef, lane);
+    lds_order();
+    return GradSum{sum, cx};
+}
+
+template <bool FULL, bool GEO>
+__device__ __forceinline__ void grad_flush(const float* rows, const GradPixels<GEO>& g, const Stage& st,
+                                           uint32_t slots, int n, int lane, float* __restrict__ gacc)
+{
+    const GradSum t = grad_sums<FULL, GEO>(rows, g, st, slots, lane);
+    const int i = grad_slot(lane);
+    const bool on = ((lane >> 1) & 3) < n && i < (GEO ? 16 : 11) && !(FULL && (i == 2 || i == 3));
+    if (on) unsafeAtomicAdd(gacc + (size_t)t.cx * 16 + i, t.v);
 }
 
 // render_geo's backward inputs (reference _r backward.cu:335-347)
@@ -3379,150 +3552,27 @@ __device__ void bwd_schedule_block(unsigned x, unsigned gx, unsigned gy, unsigne
     }
 }
 
-// The split path's backward over a 16x8 half tile (half 0: pixel rows 0-7,
-// 1: rows 8-15) in one wave, two pixels per lane: lane l takes the pixels
-// (x0 + l % 8, y) and (x0 + 8 + l % 8, y), y = y0 + l / 8.  Each staged
-// entry is evaluated for both pixels and their twelve terms enter one wave
-// reduction (the |dmean| terms as |a| + |b| per lane), so the reduction and
-// the atomics are paid once per two pixels.  It pays when the Gaussians are
-// wide enough that an entry the wave admits usually touches both 8x8 halves
-// of the 16x8 footprint: the blocks take it when a Gaussian has
-// TWO_PX_MIN_INSTANCES tile instances or more on average (two_px_lanes).
-// Measured: config 1 (R / L = 55) 0.402 -> 0.366 ms, config 2 (R / L = 7.2)
-// 0.651 -> 0.727 ms; a model of the two walks' admitted entries puts the
-// break-even at R / L ~ 24 on both scene families.
-constexpr uint64_t TWO_PX_MIN_INSTANCES = 24;
-
-__device__ __forceinline__ bool two_px_lanes(const uint32_t* __restrict__ meta)
-{
-    const uint64_t R = (uint64_t)meta[2] | ((uint64_t)meta[3] << 32), L = meta[4];
-    return R >= TWO_PX_MIN_INSTANCES * L;
-}
-
-__device__ __forceinline__ void bwd_half_tile(int W, int H, unsigned gx, unsigned tile, unsigned half,
-                                              const uint2* __restrict__ ranges, const uint32_t* __restrict__ clist,
-                                              const float4* __restrict__ rec, const float* __restrict__ bg,
-                                              const float* __restrict__ final_T,
-                                              const uint32_t* __restrict__ n_contrib_px,
-                                              const float* __restrict__ dL_dpixels, float* __restrict__ gacc,
-                                              Stage& st)
-{
-    const unsigned tx = tile % gx, ty = tile / gx;
-    const int lane = threadIdx.x;
-    const int qx = (int)tx * 16, qy = (int)ty * 16 + (int)half * 8;
-    const int pxa = qx + (lane & 7), pxb = pxa + 8, py = qy + (lane >> 3);
-    const bool ina = pxa < W && py < H, inb = pxb < W && py < H;
-    const size_t pida = (size_t)py * W + pxa, pidb = pida + 8;
-    const size_t HW = (size_t)H * W;
-    const float Tfa = ina ? final_T[pida] : 0.f, Tfb = inb ? final_T[pidb] : 0.f;
-    const int lasta = ina ? (int)n_contrib_px[pida] : 0, lastb = inb ? (int)n_contrib_px[pidb] : 0;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, b0 = 0.f, b1 = 0.f, b2 = 0.f;
-    if (ina) { a0 = dL_dpixels[pida]; a1 = dL_dpixels[HW + pida]; a2 = dL_dpixels[2 * HW + pida]; }
-    if (inb) { b0 = dL_dpixels[pidb]; b1 = dL_dpixels[HW + pidb]; b2 = dL_dpixels[2 * HW + pidb]; }
-    const int maxlast = gs::wave_max_i(max(lasta, lastb));
-    if (maxlast == 0) return;
-
-    const uint32_t* list = clist + ranges[tile].x;
-    const float qx0 = (float)qx, qy0 = (float)qy;
-    const float bga = bg[0] * a0 + bg[1] * a1 + bg[2] * a2, bgb = bg[0] * b0 + bg[1] * b1 + bg[2] * b2;
-    const BwdConst ka{(float)pxa, (float)py, a0, a1, a2, -Tfa * bga, lasta};
-    const BwdConst kb{(float)pxb, (float)py, b0, b1, b2, -Tfb * bgb, lastb};
-    const int my_k = gs::wave_sum12_index(lane);
-    BwdPixel pa{Tfa, 0.f, 0.f, 0.f}, pb{Tfb, 0.f, 0.f, 0.f};
-
-    // the same walk and software pipeline as the 8x8 quadrant waves
-    uint32_t id_cur = maxlast - 1 - lane >= 0 ? list[maxlast - 1 - lane] : 0u;
-    uint32_t id_nxt = maxlast - 65 - lane >= 0 ? list[maxlast - 65 - lane] : 0u;
-    Rec r_cur{};
-    if (maxlast - 1 - lane >= 0) r_cur = load_rec<false>(rec, id_cur);
-
-    for (int top = maxlast; top > 0; top -= 64) {
-        const int k = top - 1 - lane;
-        Rec r_nxt{};
-        uint32_t id_nn = 0;
-        if (k - 64 >= 0) r_nxt = load_rec<false>(rec, id_nxt);
-        if (k - 128 >= 0) id_nn = list[k - 128];
-        // the staging cull tests the rectangle of both halves' pixels whose
-        // last contributor lies past top - 64 (one of the two sets is not empty)
-        const int thr = max(top - 64, 0);
-        const uint64_t ma = gs::ballot(lasta > thr), mb = gs::ballot(lastb > thr);
-        float cx0 = 3.0e38f, cy0 = 3.0e38f, cx1 = -3.0e38f, cy1 = -3.0e38f;
-        if (ma != 0) active_rect(ma, qx0, qy0, cx0, cy0, cx1, cy1);
-        if (mb != 0) {
-            float x0, y0, x1, y1;
-            active_rect(mb, qx0 + 8.f, qy0, x0, y0, x1, y1);
-            cx0 = __builtin_fminf(cx0, x0);
-            cy0 = __builtin_fminf(cy0, y0);
-            cx1 = __builtin_fmaxf(cx1, x1);
-            cy1 = __builtin_fmaxf(cy1, y1);
-        }
-        const bool keep = k >= 0 && rec_may_touch(r_cur, cx0, cy0, cx1, cy1);
-        const uint64_t km = gs::ballot(keep);
-        if (keep) stage_put(st, gs::rank_below(km), r_cur, id_cur, k);
-        __syncthreads();
-        const int cnt = (int)__builtin_popcountll(km);
-        for (int j = 0; j < cnt; j++) {
-            const float4 A = st.a[j];
-            const float4 B = st.b[j];
-            const float4 Cc = st.c[j];
-            const BwdEval ea = bwd_eval(ka, A, B, Cc);
-            const BwdEval eb = bwd_eval(kb, A, B, Cc);
-            if (gs::ballot(ea.valid || eb.valid) == 0) continue;
-            float va[12], vb[12], v[12];
-            bwd_apply<false>(pa, ka, A, B, Cc, ea, va);
-            bwd_apply<false>(pb, kb, A, B, Cc, eb, vb);
-#pragma unroll
-            for (int q = 0; q < 11; q++) v[q] = va[q] + vb[q];
-            v[2] = __builtin_fabsf(va[2]) + __builtin_fabsf(vb[2]);
-            v[3] = __builtin_fabsf(va[3]) + __builtin_fabsf(vb[3]);
-            v[11] = va[11];   // never read back
-            const uint32_t cx = __builtin_amdgcn_readfirstlane(__float_as_uint(Cc.y));
-            const float tot = gs::wave_sum12<true>(v);
-            if (my_k >= 0 && my_k < 11) unsafeAtomicAdd(gacc + (size_t)cx * 16 + my_k, tot);
-        }
-        __syncthreads();
-        r_cur = r_nxt;
-        id_cur = id_nxt;
-        id_nxt = id_nn;
-    }
-}
-
 // FULL: the full-image path's rule (reference _f backward.cu:560-566): no
 // conic or opacity gradient from a pixel where opacity * G > 0.99 (the alpha
-// clamp is active); |dL/dmean2D| is accumulated but not written out.
+// clamp is active), and no |dL/dmean2D|.
 // GEO: render_geo (reference _r backward.cu:393-405,427-432,476-490): the five
 // maps enter dL/dalpha beside the colour, and their gradients
 // alpha T dL/dmap go to accumulator slots 11..15.
-// The split path without render_geo (!FULL && !GEO) walks 16x8 half tiles
-// instead of quadrants when the scene's Gaussians are wide (two_px_lanes,
-// from the forward's counts in meta; block-uniform).  Occupancy: six waves
-// per SIMD (80 VGPRs) except with render_geo's map terms.
+// Occupancy: six waves per SIMD (80 VGPRs, 6.3 KB of LDS) except with
+// render_geo's map terms.
 template <bool FULL, bool GEO>
 __device__ __forceinline__ void render_bwd_body(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, const float* __restrict__ final_T, const uint32_t* __restrict__ n_contrib_px,
     const float* __restrict__ dL_dpixels, float* __restrict__ gacc, const GeoBwd& G,
-    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, const uint32_t* __restrict__ meta,
-    Stage& st)
+    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, Stage& st, float* rows)
 {
     unsigned tile, quad, tx, ty;
     if (sched != nullptr) {
-        // bwd_schedule_kernel's order: XCD b % 8 takes its tiles heaviest first,
-        // four quadrant waves per tile (or two half-tile waves: the grid's
-        // other half of the blocks then has nothing to do)
+        // bwd_schedule_block's order: XCD b % 8 takes its tiles heaviest first,
+        // four quadrant waves per tile
         const unsigned xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-        if constexpr (!FULL && !GEO) {
-            if (two_px_lanes(meta)) {
-                const unsigned i = slot >> 1;
-                if (i >= scnt[xcd]) return;
-                const unsigned t = sched[(size_t)xcd * sched_cap(NS) + i];
-                if (cl != nullptr && !cl[t]) return;
-                bwd_half_tile(W, H, gx, t, slot & 1u, ranges, clist, rec, bg, final_T, n_contrib_px, dL_dpixels,
-                              gacc, st);
-                return;
-            }
-        }
         const unsigned i = slot >> 2;
         if (i >= scnt[xcd]) return;
         quad = slot & 3u;
@@ -3550,7 +3600,7 @@ __device__ __forceinline__ void render_bwd_body(
     // render_geo: the pixel's map gradients, plus the plane depth's
     // D = M4 / -(n . ray + 1e-8) through n = M0..2 and M4 (the ray as the
     // reference's backward takes it: (x - W / 2) / fx in double)
-    [[maybe_unused]] float dm[NUM_MAPS] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    float dm[NUM_MAPS] = {0.f, 0.f, 0.f, 0.f, 0.f};
     if constexpr (GEO) {
         if (inside) {
             for (int c = 0; c < NUM_MAPS; c++) dm[c] = G.dL_dmaps[c * HW + pid];
@@ -3575,23 +3625,21 @@ __device__ __forceinline__ void render_bwd_body(
     const float bg_dot = bg[0] * dp0 + bg[1] * dp1 + bg[2] * dp2;
     // nT_bg: the background term of dL/dalpha, before 1/(1-alpha)
     const BwdConst kc{(float)px, (float)py, dp0, dp1, dp2, -T_final * bg_dot, last};
-    // after the wave reduction this lane holds the total of gradient term
-    // my_k (accumulator slot), or nothing (my_k < 0)
-    const int my_k = gs::wave_sum12_index(lane);
-    BwdPixel px_st{T_final, 0.f, 0.f, 0.f};
+    const GradPixels<GEO> gp = grad_pixels<GEO>(rows, lane, qx0, qy0, dp0, dp1, dp2, dm);
+    BwdPixel px_st{T_final, 0.f};
 
-    // walk positions maxlast-1 .. 0 of the tile's list, back to front, with
-    // the same software pipeline as the forward
+    // walk positions maxlast-1 .. 0 of the tile's list, back to front; the
+    // next batches' list entries are in flight while one blends.  Their
+    // records are not: those registers are worth more as a sixth wave per
+    // SIMD without spills (530 -> 510 us at 6M aerial Gaussians, 1600x1066)
     uint32_t id_cur = maxlast - 1 - lane >= 0 ? list[maxlast - 1 - lane] : 0u;
     uint32_t id_nxt = maxlast - 65 - lane >= 0 ? list[maxlast - 65 - lane] : 0u;
-    Rec r_cur{};
-    if (maxlast - 1 - lane >= 0) r_cur = load_rec<GEO>(rec, id_cur);
 
     for (int top = maxlast; top > 0; top -= 64) {
         const int k = top - 1 - lane;
-        Rec r_nxt{};
+        Rec r_cur{};
         uint32_t id_nn = 0;
-        if (k - 64 >= 0) r_nxt = load_rec<GEO>(rec, id_nxt);
+        if (k >= 0) r_cur = load_rec<GEO>(rec, id_cur);
         if (k - 128 >= 0) id_nn = list[k - 128];
         // stage positions top-1, top-2, ..., top-64, keeping only Gaussians
         // that can reach a pixel whose last contributor lies past top-64
@@ -3611,56 +3659,47 @@ __device__ __forceinline__ void render_bwd_body(
         }
         __syncthreads();
         const int cnt = (int)__builtin_popcountll(km);
+        int n = 0;   // filled slots of the next contraction
+        uint32_t slots = 0u;
         for (int j = 0; j < cnt; j++) {
             const float4 A = st.a[j];
             const float4 B = st.b[j];
             const float4 Cc = st.c[j];
             const BwdEval e = bwd_eval(kc, A, B, Cc);
             if (gs::ballot(e.valid) == 0) continue;   // no lane blends the entry: nothing changes
-            float vals[12];
+            float m_dp = 0.f;
             if constexpr (GEO) {
-                float mv[NUM_MAPS];
-                for (int c = 0; c < NUM_MAPS; c++) mv[c] = st_map[c * 64 + j];
-                float m_dp = mv[0] * dm[0];
-                for (int c = 1; c < NUM_MAPS; c++) m_dp = __builtin_fmaf(mv[c], dm[c], m_dp);
-                const float dcc = bwd_apply<FULL, true>(px_st, kc, A, B, Cc, e, vals, m_dp);
-                const uint32_t cx = __builtin_amdgcn_readfirstlane(__float_as_uint(Cc.y));
-                // slot 11: the first map's gradient; the other four in a
-                // second reduction, into slots 12..15
-                vals[11] = dcc * dm[0];
-                float v2[12] = {dcc * dm[1], dcc * dm[2], dcc * dm[3], dcc * dm[4], 0.f, 0.f,
-                                0.f,         0.f,         0.f,         0.f,         0.f, 0.f};
-                const float tot = gs::wave_sum12<true>(vals);
-                const float tot2 = gs::wave_sum12<false>(v2);
-                if (my_k >= 0) unsafeAtomicAdd(gacc + (size_t)cx * 16 + my_k, tot);
-                if (my_k >= 0 && my_k < 4) unsafeAtomicAdd(gacc + (size_t)cx * 16 + 12 + my_k, tot2);
-            } else {
-                bwd_apply<FULL>(px_st, kc, A, B, Cc, e, vals);
-                const uint32_t cx = __builtin_amdgcn_readfirstlane(__float_as_uint(Cc.y));   // one Gaussian per entry
-                const float tot = gs::wave_sum12<true>(vals);
-                // the eleven totals of one Gaussian land in one 64-byte accumulator
-                if (my_k >= 0 && my_k < 11) unsafeAtomicAdd(gacc + (size_t)cx * 16 + my_k, tot);
+                m_dp = st_map[j] * dm[0];
+                for (int c = 1; c < NUM_MAPS; c++) m_dp = __builtin_fmaf(st_map[c * 64 + j], dm[c], m_dp);
+            }
+            grad_put(rows, n, lane, bwd_apply<FULL, GEO>(px_st, kc, A, B, Cc, e, m_dp));
+            slots |= (uint32_t)j << (8 * n);
+            if (++n == GRAD_SLOTS) {
+                grad_flush<FULL, GEO>(rows, gp, st, slots, n, lane, gacc);
+                n = 0;
+                slots = 0u;
             }
         }
+        // the staged entries go with the batch
+        if (n > 0) grad_flush<FULL, GEO>(rows, gp, st, slots, n, lane, gacc);
         __syncthreads();
-        r_cur = r_nxt;
         id_cur = id_nxt;
         id_nxt = id_nn;
     }
 }
 
 template <bool FULL, bool GEO = false>
-__global__ __launch_bounds__(64, GEO ? 5 : 6) void render_bwd_kernel(
+__global__ __launch_bounds__(64, GEO ? 4 : 6) void render_bwd_kernel(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, const float* __restrict__ final_T, const uint32_t* __restrict__ n_contrib_px,
     const float* __restrict__ dL_dpixels, float* __restrict__ gacc, GeoBwd G,
-    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, const uint32_t* __restrict__ meta,
-    ClearBuf clr)
+    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, ClearBuf clr)
 {
     __shared__ Stage st;
+    __shared__ __align__(16) float rows[GRAD_SLOTS * GRAD_STRIDE];
     render_bwd_body<FULL, GEO>(W, H, gx, gy, sgx, NS, ranges, clist, rec, cl, bg, final_T, n_contrib_px, dL_dpixels,
-                               gacc, G, sched, scnt, meta, st);
+                               gacc, G, sched, scnt, st, rows);
     clear_share(clr);
 }
 
@@ -3671,7 +3710,7 @@ __global__ __launch_bounds__(256) void clear_kernel(ClearBuf clr)
 }
 
 // ---- VALU probes: the blend kernels' per-entry arithmetic (fwd_blend_step;
-// bwd_eval + bwd_apply + wave_sum12), on 64 entries staged in LDS once, with no
+// bwd_eval + bwd_apply + grad_sums), on 64 entries staged in LDS once, with no
 // global memory traffic, in the blend kernels' 64-thread blocks.  Their VALU
 // instruction rate is the ceiling the blend kernels' rate is compared with.
 constexpr int VALU_PROBE_BLOCKS = 16384;
@@ -3721,48 +3760,28 @@ __global__ __launch_bounds__(64) void valu_probe_kernel(int iters, float* __rest
             out += p.C0 + p.C1 + p.C2 + p.T + (float)(p.last + p.n2l);
         }
         out += (float)observed;
-    } else if (WHICH == 2) {
-        // the backward's half-tile walk (bwd_half_tile): two pixels per lane
-        // (here at one position, so that both blend every entry), one
-        // reduction per entry, the atomics replaced by a sum
-        const int my_k = gs::wave_sum12_index(lane);
-        const BwdConst ka{pxf, pyf, 0.3f, -0.2f, 0.1f, -0.05f, 64};
-        const BwdConst kb{pxf, pyf, -0.1f, 0.25f, 0.2f, -0.04f, 64};
-        for (int it = 0; it < iters; it++) {
-            BwdPixel pa{0.2f, 0.f, 0.f, 0.f}, pb{0.25f, 0.f, 0.f, 0.f};
-            for (int j = 0; j < 64; j++) {
-                const float4 A = st.a[j], B = st.b[j], Cc = st.c[j];
-                const BwdEval ea = bwd_eval(ka, A, B, Cc);
-                const BwdEval eb = bwd_eval(kb, A, B, Cc);
-                if (gs::ballot(ea.valid || eb.valid) == 0) continue;
-                float va[12], vb[12], v[12];
-                bwd_apply<false>(pa, ka, A, B, Cc, ea, va);
-                bwd_apply<false>(pb, kb, A, B, Cc, eb, vb);
-#pragma unroll
-                for (int q = 0; q < 11; q++) v[q] = va[q] + vb[q];
-                v[2] = __builtin_fabsf(va[2]) + __builtin_fabsf(vb[2]);
-                v[3] = __builtin_fabsf(va[3]) + __builtin_fabsf(vb[3]);
-                v[11] = va[11];
-                const float tot = gs::wave_sum12<true>(v);
-                if (my_k >= 0 && my_k < 11 && tot != 0.f) out += tot;
-            }
-            out += pa.T + pb.T;
-        }
     } else {
         // the backward: render_bwd_kernel's entry loop, the accumulator
         // atomics replaced by a sum
-        const int my_k = gs::wave_sum12_index(lane);
+        __shared__ __align__(16) float rows[GRAD_SLOTS * GRAD_STRIDE];
         const BwdConst kc{pxf, pyf, 0.3f, -0.2f, 0.1f, -0.05f, 64};
+        const float dm[NUM_MAPS] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        const GradPixels<false> gp = grad_pixels<false>(rows, lane, 0.f, 0.f, kc.dp0, kc.dp1, kc.dp2, dm);
         for (int it = 0; it < iters; it++) {
-            BwdPixel p{0.2f, 0.f, 0.f, 0.f};
+            BwdPixel p{0.2f, 0.f};
+            int n = 0;
+            uint32_t slots = 0u;
             for (int j = 0; j < 64; j++) {
                 const float4 A = st.a[j], B = st.b[j], Cc = st.c[j];
                 const BwdEval e = bwd_eval(kc, A, B, Cc);
                 if (gs::ballot(e.valid) == 0) continue;
-                float vals[12];
-                bwd_apply<false>(p, kc, A, B, Cc, e, vals);
-                const float tot = gs::wave_sum12<true>(vals);
-                if (my_k >= 0 && my_k < 11 && tot != 0.f) out += tot;
+                grad_put(rows, n, lane, bwd_apply<false>(p, kc, A, B, Cc, e));
+                slots |= (uint32_t)j << (8 * n);
+                if (++n == GRAD_SLOTS) {
+                    out += grad_sums<false, false>(rows, gp, st, slots, lane).v;
+                    n = 0;
+                    slots = 0u;
+                }
             }
             out += p.T;
         }
@@ -4315,19 +4334,19 @@ int render_backward_impl(bool full, int P, int64_t R, int W, int H, const float*
                      hipLaunchKernelGGL(render_bwd_kernel<true>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
                                         NS, rng, clist, recs, compute_locally, bg, at<float>(img, il.final_T),
                                         at<uint32_t>(img, il.n_contrib), dL_dpixels, reinterpret_cast<float*>(gacc),
-                                        GeoBwd{}, nullptr, nullptr, nullptr, ClearBuf{nullptr, 0}));
+                                        GeoBwd{}, nullptr, nullptr, ClearBuf{nullptr, 0}));
         } else if (geo != nullptr) {
             GS_TIMED("render_bwd_geo_kernel", stream,
                      hipLaunchKernelGGL((render_bwd_kernel<false, true>), dim3(nblk), dim3(64), 0, stream, W, H, gx,
                                         gy, sgx, NS, rng, clist, recs, compute_locally, bg,
                                         at<float>(img, il.final_T), at<uint32_t>(img, il.n_contrib), dL_dpixels,
-                                        reinterpret_cast<float*>(gacc), *geo, sched, scnt, nullptr, clr));
+                                        reinterpret_cast<float*>(gacc), *geo, sched, scnt, clr));
         } else {
             GS_TIMED("render_bwd_kernel", stream,
                      hipLaunchKernelGGL(render_bwd_kernel<false>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
                                         NS, rng, clist, recs, compute_locally, bg, at<float>(img, il.final_T),
                                         at<uint32_t>(img, il.n_contrib), dL_dpixels, reinterpret_cast<float*>(gacc),
-                                        GeoBwd{}, sched, scnt, at<const uint32_t>(geom, g.meta), clr));
+                                        GeoBwd{}, sched, scnt, clr));
         }
         GS_LAUNCH_CHECK("render_bwd_kernel");
     } else if (clr.n16 != 0) {
@@ -4721,18 +4740,15 @@ namespace gs {
 // entries per wave, VALU_PROBE_BLOCKS waves.
 int render_valu_probe(int which, int iters, float* y, hipStream_t stream)
 {
-    GS_REQUIRE(which >= 0 && which <= 2, "which must be 0 (forward), 1 (backward) or 2 (backward, half tiles)");
+    GS_REQUIRE(which >= 0 && which <= 2, "which must be 0 (forward), 1 or 2 (backward)");
     GS_REQUIRE(iters >= 0 && y != nullptr, "iters must be >= 0 and y non-null");
     if (iters == 0) return GS_OK;
     if (which == 0) {
         GS_TIMED("valu_probe_fwd_kernel", stream,
                  hipLaunchKernelGGL(valu_probe_kernel<0>, dim3(VALU_PROBE_BLOCKS), dim3(64), 0, stream, iters, y));
-    } else if (which == 1) {
+    } else {
         GS_TIMED("valu_probe_bwd_kernel", stream,
                  hipLaunchKernelGGL(valu_probe_kernel<1>, dim3(VALU_PROBE_BLOCKS), dim3(64), 0, stream, iters, y));
-    } else {
-        GS_TIMED("valu_probe_bwd2_kernel", stream,
-                 hipLaunchKernelGGL(valu_probe_kernel<2>, dim3(VALU_PROBE_BLOCKS), dim3(64), 0, stream, iters, y));
     }
     GS_LAUNCH_CHECK("valu_probe_kernel");
     return GS_OK;
