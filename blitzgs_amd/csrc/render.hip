@@ -2653,12 +2653,9 @@ struct FwdOut {
 };
 
 template <int MODE>
-// (Waves per SIMD.  The split path's walk: seven (72 VGPRs; one 8-byte value
-// spilled around the loop, none inside it): measured 2.5 % faster than six,
-// and six was 3 % faster than the 84 VGPRs the compiler picks unbounded;
-// eight force spills inside the loop and were slower.  The other paths: six;
-// the fused render_geo walk carries five more accumulators: five, no spills.)
-__global__ __launch_bounds__(64, MODE == BLEND_SPLIT ? 7 : (MODE == BLEND_SPLIT_GEO ? 5 : 6)) void render_fwd_kernel(
+// (waves per SIMD: eight fit in 64 VGPRs without spills in the loop;
+// render_geo's maps and their LDS leave six or seven)
+__global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, FwdOut O)
@@ -2701,20 +2698,20 @@ __global__ __launch_bounds__(64, MODE == BLEND_SPLIT ? 7 : (MODE == BLEND_SPLIT_
     float wmax = 0.f;      // largest blend weight so far, and its Gaussian (full / simp)
     uint32_t imax = 0u;
 
-    // software pipeline: while a batch blends, the next batch's records and
-    // the list entries of the batch after it are in flight
+    // the list entries of the next two batches are in flight while one blends.
+    // Their records are not: the registers they would hold cost two waves per
+    // SIMD, which hide their latency better.  Measured: 6M aerial Gaussians at
+    // 1600x1066 272 -> 263 us (the full-image path's blend 232 -> 221 us)
     uint32_t id_cur = lane < n ? list[lane] : 0u;
     uint32_t id_nxt = 64 + lane < n ? list[64 + lane] : 0u;
-    Rec r_cur{};
-    if (lane < n) r_cur = load_rec<true>(rec, id_cur);
 
     for (int base = 0; base < n; base += 64) {
         const uint64_t live = gs::ballot(px_st.T > 0.0f);
         if (live == 0) break;
         const int k = base + lane;
-        Rec r_nxt{};
+        Rec r_cur{};
         uint32_t id_nn = 0;
-        if (k + 64 < n) r_nxt = load_rec<true>(rec, id_nxt);
+        if (k < n) r_cur = load_rec<true>(rec, id_cur);
         if (k + 128 < n) id_nn = list[k + 128];
         // stage the batch, keeping only Gaussians that can reach a pixel of
         // the quadrant that is still blending (a finished pixel takes no
@@ -2796,7 +2793,6 @@ __global__ __launch_bounds__(64, MODE == BLEND_SPLIT ? 7 : (MODE == BLEND_SPLIT_
         else
             blend_batch(std::false_type{});
         __syncthreads();
-        r_cur = r_nxt;
         id_cur = id_nxt;
         id_nxt = id_nn;
     }
