@@ -43,14 +43,14 @@
 // global atomics instead of the LDS histogram (same result after step 4).
 //
 // Blend design.  One wave64 per 8x8 quadrant of a tile, one pixel per lane,
-// no block-wide barriers: a wave stages batches of 64 list entries (their
-// records gathered while the previous batch blends) in its own LDS slots,
-// dropping those that provably cannot reach the quadrant, and stops as soon as
-// all of its 64 pixels are saturated.  The backward walks each quadrant's
-// list back to front from the largest last contributor of its pixels, reduces
-// every Gaussian's eleven gradient terms across the wave and adds them into
-// the Gaussian's 64-byte accumulator with one atomic instruction per (wave,
-// Gaussian) instead of eleven atomics per (pixel, Gaussian); a final pass
+// no block-wide barriers: a wave stages batches of 64 list entries in its own
+// LDS slots, dropping those that provably cannot reach the quadrant, marks the
+// entries that it blends, and stops as soon as all of its 64 pixels are
+// saturated.  The backward walks each quadrant's marked entries back to front
+// from the largest last contributor of its pixels, forms the eleven gradient
+// sums of four Gaussians at a time across the wave and adds them into the
+// Gaussians' 64-byte accumulators with one atomic instruction per wave and
+// four Gaussians instead of eleven atomics per (pixel, Gaussian); a final pass
 // writes the reference's gradient arrays from the accumulators.
 #include <mutex>
 
@@ -107,6 +107,7 @@ struct GeomLayout {
     // per-tile count difference grids
     size_t regmask, rcount, rstart, rcursor, rhist, rcls_count, rcls_list, grid;
     size_t qwork, sched, scnt;   // split path: per-quadrant work (forward), backward block order
+    size_t stail;                // per quadrant: the staged entries of its list's last, partial batch (StagedMasks)
     size_t total;
 };
 
@@ -165,6 +166,7 @@ GeomLayout geom_layout(int P, int W, int H)
         g.qwork = o; o = align256(o + sizeof(uint32_t) * 4 * (size_t)g.T);
         g.sched = o; o = align256(o + sizeof(uint32_t) * 8 * (size_t)sched_cap(NS));
         g.scnt = o; o = align256(o + sizeof(uint32_t) * 8);
+        g.stail = o; o = align256(o + sizeof(uint64_t) * 4 * (size_t)g.T);
     }
     g.total = o;
     return g;
@@ -189,7 +191,7 @@ ImgLayout img_layout(int W, int H)
 }
 
 struct BinLayout {
-    size_t sortkey, point_list, keys, clist, total;
+    size_t sortkey, point_list, keys, clist, smask, total;
 };
 
 // The compact list comes first: it is the only array the blend, the backward
@@ -197,7 +199,9 @@ struct BinLayout {
 // after the forward) follow it, and the forward's unsorted keys use their
 // space as scratch.  Nothing at or past an offset depends on R except through
 // that offset, so a buffer laid out for a capacity C >= R serves R: its
-// compact list is at the same place and the point list fits.
+// compact list is at the same place and the point list fits; where its staged
+// masks lie, which depends on C, the forward leaves in meta[11] (in units of
+// 256 bytes).
 BinLayout bin_layout(int64_t R)
 {
     BinLayout b;
@@ -207,6 +211,7 @@ BinLayout bin_layout(int64_t R)
     b.sortkey = o;                                   // 8R bytes inside point list + keys
     o = align256(o + sizeof(uint32_t) * (size_t)R);
     b.keys = o; o = align256(o + sizeof(uint64_t) * (size_t)R);
+    b.smask = o; o = align256(o + sizeof(uint64_t) * 4 * ((size_t)R / 64 + 1));
     b.total = o < 256 ? 256 : o;
     return b;
 }
@@ -2633,6 +2638,36 @@ struct ClearAtExit {
     __device__ ~ClearAtExit() { clear_share(c); }
 };
 
+// Which list entries the backward of a quadrant stages: one bit per list
+// position, a 64-bit word per batch of 64 positions of the tile's list, left
+// by the forward.  The split path marks the entries that a pixel takes, the
+// full-image path those its forward staged (all that can reach a pixel that
+// still blends).  The backward then neither loads the other entries' records
+// nor repeats the test that drops them, and stages 64 marked entries at a
+// time, wherever in the list they are.  Batch b of a list that starts at
+// position x of the whole compact list has, when it is full, the word of the
+// multiple of 64 that lies in it, (x + 64 b + 63) / 64, which no other batch
+// holds; a tile's last batch of fewer than 64 has a word of its own.  Written
+// at least up to the batch of the quadrant's largest last contributor.
+//
+// Why: testing an entry took the backward a sixth of its VALU instructions
+// (ten list entries are tested per blended one).  Measured at 6M aerial
+// Gaussians, 1600x1066: render backward 506 -> 422 us (449 us with the staged
+// entries marked), forward 263 -> 283 us (267 us); at 1M wide ones, 1920x1080:
+// 286 -> 260 us and 174 -> 187 us.  The evaluation views of the full-image
+// path run no backward, so that path takes the cheaper mark (forward 221 ->
+// 222 us at 6M; with the other 241 us).
+struct StagedMasks {
+    uint64_t* full;   // 4 words (quadrants) per 64 positions, in the binning buffer
+    uint64_t* tail;   // 4 words per tile
+
+    __device__ __forceinline__ uint64_t* word(unsigned tile, unsigned quad, uint32_t x, int n, int b) const
+    {
+        return 64 * (b + 1) <= n ? full + 4 * (size_t)((x + 64u * (uint32_t)b + 63u) >> 6) + quad
+                                 : tail + 4 * (size_t)tile + quad;
+    }
+};
+
 struct FwdOut {
     float* out_color;
     float* final_T;
@@ -2650,6 +2685,9 @@ struct FwdOut {
     float* out_plane_depth;        // geo: (H,W)
     float focal_x, focal_y, cx, cy;   // geo: the plane depth's pixel rays
     ClearBuf clr;                  // split: a caller's buffer cleared after the walks (none: n16 == 0)
+    StagedMasks sm;                // all but BLEND_GEO
+    uint32_t* meta;                // ... which leaves sm.full's place in meta[11]
+    uint32_t sm_off;
 };
 
 template <int MODE>
@@ -2661,6 +2699,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     const float* __restrict__ bg, FwdOut O)
 {
     [[maybe_unused]] const ClearAtExit clear_at_exit{O.clr};
+    if (MODE != BLEND_GEO && blockIdx.x == 0 && threadIdx.x == 0) O.meta[11] = O.sm_off;
     unsigned tile, quad, tx, ty;
     if (!block_to_tile(blockIdx.x, gx, gy, sgx, NS, tile, quad, tx, ty)) return;
     const int lane = threadIdx.x;
@@ -2704,8 +2743,17 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     // 1600x1066 272 -> 263 us (the full-image path's blend 232 -> 221 us)
     uint32_t id_cur = lane < n ? list[lane] : 0u;
     uint32_t id_nxt = 64 + lane < n ? list[64 + lane] : 0u;
+    // the staged masks of up to 64 batches, batch b in lane b % 64 (written
+    // together: a store in the loop would hold up its loads, which share its
+    // counter: 6 us at 6M)
+    uint32_t sm_lo = 0u, sm_hi = 0u;
+    auto put_masks = [&](int b0, int b1) {   // batches b0 .. b1 - 1, all of one word of 64
+        if (b0 + lane < b1)
+            *O.sm.word(tile, quad, range.x, n, b0 + lane) = ((uint64_t)sm_hi << 32) | sm_lo;
+    };
+    int base = 0;
 
-    for (int base = 0; base < n; base += 64) {
+    for (; base < n; base += 64) {
         const uint64_t live = gs::ballot(px_st.T > 0.0f);
         if (live == 0) break;
         const int k = base + lane;
@@ -2730,6 +2778,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
         }
         __syncthreads();
         const int cnt = (int)__builtin_popcountll(km);
+        [[maybe_unused]] uint32_t taken = 0u;   // lane j: not zero when a pixel takes staged entry j
         // Branch-free blend of one staged entry: every lane evaluates it and
         // the state changes are selects, so no exec-mask bookkeeping.  OBS
         // (split path): lane jj of obs_cnt takes the number of pixels that
@@ -2740,6 +2789,10 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
             const FwdStep f = fwd_blend_step(px_st, A, B, Cc, pxf, pyf);
             const bool upd = f.upd;
             const float wgt = f.wgt;
+            if constexpr (is_split(MODE)) {
+                const uint64_t um = gs::ballot(upd);
+                taken = gs::write_lane(taken, (uint32_t)um | (uint32_t)(um >> 32), jj);
+            }
             if constexpr (is_geo(MODE)) {
                 // the colour's update rule: a pixel that does not take the
                 // entry adds map * 0
@@ -2792,11 +2845,26 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
             blend_batch(std::integral_constant<bool, is_split(MODE)>{});
         else
             blend_batch(std::false_type{});
+        if constexpr (MODE != BLEND_GEO) {
+            uint64_t m = km;
+            if constexpr (is_split(MODE)) {
+                const uint64_t slots = gs::ballot(taken != 0u);
+                m = gs::ballot(keep && ((slots >> gs::rank_below(km)) & 1u) != 0);
+            }
+            const int b = base >> 6;
+            sm_lo = gs::write_lane(sm_lo, (uint32_t)m, b & 63);
+            sm_hi = gs::write_lane(sm_hi, (uint32_t)(m >> 32), b & 63);
+            if ((b & 63) == 63) put_masks(b - 63, b + 1);
+        }
         __syncthreads();
         id_cur = id_nxt;
         id_nxt = id_nn;
     }
 
+    if constexpr (MODE != BLEND_GEO) {
+        const int nb = base < n ? base >> 6 : (n + 63) >> 6;   // batches walked
+        put_masks(nb & ~63, nb);
+    }
     if constexpr (is_geo(MODE)) {
         // plane depth (reference _r forward.cu:411): M4 / -(M0 rx + M1 ry + M2
         // + 1e-8), the 1e-8 a double literal there: the sum in float, the rest
@@ -3304,7 +3372,7 @@ __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, co
 // cycles, of either alone 34 and 71; a bf16 MFMA does overlap, but splitting
 // the rows into three bf16 parts costs more VALU than it saves); eight entries
 // of eight pixels per lane (fewer instructions, but four waves per SIMD and
-// twice the accumulator lines per entry): 508 -> 594 us at 6M.
+// twice the accumulator lines per entry): 422 -> 508 us at 6M.
 constexpr int GRAD_SLOTS = 4;          // entries per flush
 constexpr int GRAD_STRIDE = 3 * 64 + 8;   // floats per slot: 3 rows, and 8 more so that 8 lanes' 16-byte reads meet 32 banks
 
@@ -3394,11 +3462,11 @@ struct GradSum {
     uint32_t cx;   // of this accumulator row
 };
 
-// The sums of the slots' entries; byte e of `slots` is the staged position of
-// slot e's entry.  grad_flush adds the first n slots' to the accumulators.
+// The sums of the four entries staged from j0 on.  grad_flush adds the first
+// n of them to the accumulators.
 template <bool FULL, bool GEO>
 __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels<GEO>& g, const Stage& st,
-                                             uint32_t slots, int lane)
+                                             int j0, int lane)
 {
     lds_order();
     const int e = (lane >> 1) & 3;
@@ -3406,7 +3474,7 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
     const float4 w = *reinterpret_cast<const float4*>(r);
     const float4 v = *reinterpret_cast<const float4*>(r + 64);
     const float4 u = *reinterpret_cast<const float4*>(r + 128);
-    const int j = (int)((slots >> (8 * e)) & 63u);
+    const int j = j0 + e;
     const float4 A = st.a[j];
     const float2 B = *reinterpret_cast<const float2*>(&st.b[j]);
     const uint32_t cx = __float_as_uint(st.c[j].y);
@@ -3447,9 +3515,9 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
 
 template <bool FULL, bool GEO>
 __device__ __forceinline__ void grad_flush(const float* rows, const GradPixels<GEO>& g, const Stage& st,
-                                           uint32_t slots, int n, int lane, float* __restrict__ gacc)
+                                           int j0, int n, int lane, float* __restrict__ gacc)
 {
-    const GradSum t = grad_sums<FULL, GEO>(rows, g, st, slots, lane);
+    const GradSum t = grad_sums<FULL, GEO>(rows, g, st, j0, lane);
     const int i = grad_slot(lane);
     const bool on = ((lane >> 1) & 3) < n && i < (GEO ? 16 : 11) && !(FULL && (i == 2 || i == 3));
     if (on) unsafeAtomicAdd(gacc + (size_t)t.cx * 16 + i, t.v);
@@ -3562,7 +3630,7 @@ __device__ __forceinline__ void render_bwd_body(
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, const float* __restrict__ final_T, const uint32_t* __restrict__ n_contrib_px,
     const float* __restrict__ dL_dpixels, float* __restrict__ gacc, const GeoBwd& G,
-    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, Stage& st, float* rows)
+    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, StagedMasks sm, Stage& st, float* rows)
 {
     unsigned tile, quad, tx, ty;
     if (sched != nullptr) {
@@ -3616,7 +3684,9 @@ __device__ __forceinline__ void render_bwd_body(
 
     __shared__ float st_map[GEO ? NUM_MAPS * 64 : 1];
 
-    const uint32_t* list = clist + ranges[tile].x;
+    const uint2 range = ranges[tile];
+    const uint32_t* list = clist + range.x;
+    const int n_list = (int)(range.y - range.x);
     const float qx0 = (float)qx, qy0 = (float)qy;
     const float bg_dot = bg[0] * dp0 + bg[1] * dp1 + bg[2] * dp2;
     // nT_bg: the background term of dL/dalpha, before 1/(1-alpha)
@@ -3624,63 +3694,76 @@ __device__ __forceinline__ void render_bwd_body(
     const GradPixels<GEO> gp = grad_pixels<GEO>(rows, lane, qx0, qy0, dp0, dp1, dp2, dm);
     BwdPixel px_st{T_final, 0.f};
 
-    // walk positions maxlast-1 .. 0 of the tile's list, back to front; the
-    // next batches' list entries are in flight while one blends.  Their
-    // records are not: those registers are worth more as a sixth wave per
-    // SIMD without spills (530 -> 510 us at 6M aerial Gaussians, 1600x1066)
-    uint32_t id_cur = maxlast - 1 - lane >= 0 ? list[maxlast - 1 - lane] : 0u;
-    uint32_t id_nxt = maxlast - 65 - lane >= 0 ? list[maxlast - 65 - lane] : 0u;
-
-    for (int top = maxlast; top > 0; top -= 64) {
-        const int k = top - 1 - lane;
-        Rec r_cur{};
-        uint32_t id_nn = 0;
-        if (k >= 0) r_cur = load_rec<GEO>(rec, id_cur);
-        if (k - 128 >= 0) id_nn = list[k - 128];
-        // stage positions top-1, top-2, ..., top-64, keeping only Gaussians
-        // that can reach a pixel whose last contributor lies past top-64
-        // (the other pixels blend no entry of this batch); that pixel set is
-        // never empty: it holds the pixels of the largest last contributor
-        float cx0, cy0, cx1, cy1;
-        active_rect(gs::ballot(last > max(top - 64, 0)), qx0, qy0, cx0, cy0, cx1, cy1);
-        const bool keep = k >= 0 && rec_may_touch(r_cur, cx0, cy0, cx1, cy1);
-        const uint64_t km = gs::ballot(keep);
-        if (keep) stage_put(st, gs::rank_below(km), r_cur, id_cur, k);
-        if constexpr (GEO) {
-            if (keep) {
-                const int slot = gs::rank_below(km);
-                const float* m = G.all_map + (size_t)NUM_MAPS * r_cur.gid;
-                for (int c = 0; c < NUM_MAPS; c++) st_map[c * 64 + slot] = m[c];
+    // Walks the staged positions from the largest last contributor back to the
+    // list's start: the words of the staged masks (64 of them at a time in the
+    // lanes of mw) are unpacked into a queue of positions, last first, until
+    // 64 are there or the words are used up, and those entries are staged
+    // together.  The queue lies in the row buffer, which is free then.
+    uint32_t* queue = reinterpret_cast<uint32_t*>(rows);
+    static_assert(GRAD_SLOTS * GRAD_STRIDE >= 128, "the queue holds up to 127 positions");
+    int b = (maxlast - 1) >> 6, held = 64;
+    uint64_t mw = 0;
+    uint32_t rest_pos = 0;   // the positions left over from the last unpacking, one per lane
+    int rest = 0;
+    for (;;) {
+        int cnt = rest;
+        if (lane < rest) queue[lane] = rest_pos;
+        while (cnt < 64 && b >= 0) {
+            if (held == 64) {
+                mw = b >= lane ? *sm.word(tile, quad, range.x, n_list, b - lane) : 0ull;
+                held = 0;
             }
+            const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)mw, held);
+            const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(mw >> 32), held);
+            const uint64_t m = __builtin_bitreverse64(((uint64_t)hi << 32) | lo);   // bit l: position 64 b + 63 - l
+            if ((m >> lane) & 1u) queue[cnt + gs::rank_below(m)] = (uint32_t)(64 * b + 63 - lane);
+            cnt += (int)__builtin_popcountll(m);
+            b--;
+            held++;
         }
-        __syncthreads();
-        const int cnt = (int)__builtin_popcountll(km);
-        int n = 0;   // filled slots of the next contraction
-        uint32_t slots = 0u;
-        for (int j = 0; j < cnt; j++) {
-            const float4 A = st.a[j];
-            const float4 B = st.b[j];
-            const float4 Cc = st.c[j];
-            const BwdEval e = bwd_eval(kc, A, B, Cc);
-            if (gs::ballot(e.valid) == 0) continue;   // no lane blends the entry: nothing changes
-            float m_dp = 0.f;
+        if (cnt == 0) break;
+        rest = max(cnt - 64, 0);
+        cnt = min(cnt, 64);
+        lds_order();
+        const uint32_t pos = queue[lane];
+        if (lane < rest) rest_pos = queue[64 + lane];
+        lds_order();
+        if (lane < cnt) {
+            const uint32_t id = list[pos];
+            const Rec r = load_rec<GEO>(rec, id);
+            stage_put(st, lane, r, id, (int)pos);
             if constexpr (GEO) {
-                m_dp = st_map[j] * dm[0];
-                for (int c = 1; c < NUM_MAPS; c++) m_dp = __builtin_fmaf(st_map[c * 64 + j], dm[c], m_dp);
+                const float* m = G.all_map + (size_t)NUM_MAPS * r.gid;
+                for (int c = 0; c < NUM_MAPS; c++) st_map[c * 64 + lane] = m[c];
             }
-            grad_put(rows, n, lane, bwd_apply<FULL, GEO>(px_st, kc, A, B, Cc, e, m_dp));
-            slots |= (uint32_t)j << (8 * n);
-            if (++n == GRAD_SLOTS) {
-                grad_flush<FULL, GEO>(rows, gp, st, slots, n, lane, gacc);
-                n = 0;
-                slots = 0u;
+        } else if (lane < ((cnt + GRAD_SLOTS - 1) & ~(GRAD_SLOTS - 1))) {
+            // the last group's empty slots: an entry that no pixel blends
+            st.a[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+            st.b[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+            st.c[lane] = make_float4(0.f, 0.f, 0.f, __builtin_huge_valf());
+            if constexpr (GEO) {
+                for (int c = 0; c < NUM_MAPS; c++) st_map[c * 64 + lane] = 0.f;
             }
         }
-        // the staged entries go with the batch
-        if (n > 0) grad_flush<FULL, GEO>(rows, gp, st, slots, n, lane, gacc);
         __syncthreads();
-        id_cur = id_nxt;
-        id_nxt = id_nn;
+        for (int j0 = 0; j0 < cnt; j0 += GRAD_SLOTS) {
+#pragma unroll
+            for (int s = 0; s < GRAD_SLOTS; s++) {
+                const int j = j0 + s;
+                const float4 A = st.a[j];
+                const float4 B = st.b[j];
+                const float4 Cc = st.c[j];
+                const BwdEval e = bwd_eval(kc, A, B, Cc);
+                float m_dp = 0.f;
+                if constexpr (GEO) {
+                    m_dp = st_map[j] * dm[0];
+                    for (int c = 1; c < NUM_MAPS; c++) m_dp = __builtin_fmaf(st_map[c * 64 + j], dm[c], m_dp);
+                }
+                grad_put(rows, s, lane, bwd_apply<FULL, GEO>(px_st, kc, A, B, Cc, e, m_dp));
+            }
+            grad_flush<FULL, GEO>(rows, gp, st, j0, cnt - j0, lane, gacc);
+        }
+        __syncthreads();
     }
 }
 
@@ -3690,12 +3773,15 @@ __global__ __launch_bounds__(64, GEO ? 4 : 6) void render_bwd_kernel(
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, const float* __restrict__ final_T, const uint32_t* __restrict__ n_contrib_px,
     const float* __restrict__ dL_dpixels, float* __restrict__ gacc, GeoBwd G,
-    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, ClearBuf clr)
+    const uint32_t* __restrict__ sched, const uint32_t* __restrict__ scnt, uint64_t* stail, char* binning,
+    const uint32_t* __restrict__ meta, ClearBuf clr)
 {
     __shared__ Stage st;
     __shared__ __align__(16) float rows[GRAD_SLOTS * GRAD_STRIDE];
     render_bwd_body<FULL, GEO>(W, H, gx, gy, sgx, NS, ranges, clist, rec, cl, bg, final_T, n_contrib_px, dL_dpixels,
-                               gacc, G, sched, scnt, st, rows);
+                               gacc, G, sched, scnt,
+                               StagedMasks{reinterpret_cast<uint64_t*>(binning + 256 * (size_t)meta[11]), stail}, st,
+                               rows);
     clear_share(clr);
 }
 
@@ -3765,19 +3851,14 @@ __global__ __launch_bounds__(64) void valu_probe_kernel(int iters, float* __rest
         const GradPixels<false> gp = grad_pixels<false>(rows, lane, 0.f, 0.f, kc.dp0, kc.dp1, kc.dp2, dm);
         for (int it = 0; it < iters; it++) {
             BwdPixel p{0.2f, 0.f};
-            int n = 0;
-            uint32_t slots = 0u;
-            for (int j = 0; j < 64; j++) {
-                const float4 A = st.a[j], B = st.b[j], Cc = st.c[j];
-                const BwdEval e = bwd_eval(kc, A, B, Cc);
-                if (gs::ballot(e.valid) == 0) continue;
-                grad_put(rows, n, lane, bwd_apply<false>(p, kc, A, B, Cc, e));
-                slots |= (uint32_t)j << (8 * n);
-                if (++n == GRAD_SLOTS) {
-                    out += grad_sums<false, false>(rows, gp, st, slots, lane).v;
-                    n = 0;
-                    slots = 0u;
+            for (int j0 = 0; j0 < 64; j0 += GRAD_SLOTS) {
+#pragma unroll
+                for (int s = 0; s < GRAD_SLOTS; s++) {
+                    const float4 A = st.a[j0 + s], B = st.b[j0 + s], Cc = st.c[j0 + s];
+                    const BwdEval e = bwd_eval(kc, A, B, Cc);
+                    grad_put(rows, s, lane, bwd_apply<false>(p, kc, A, B, Cc, e));
                 }
+                out += grad_sums<false, false>(rows, gp, st, j0, lane).v;
             }
             out += p.T;
         }
@@ -4246,6 +4327,9 @@ int render_forward_impl(int mode, int P, int64_t R, int W, int H, const float* b
     O.n_contrib_px = at<uint32_t>(img, il.n_contrib);
     O.n_contrib2loss_px = at<uint32_t>(img, il.n_contrib2loss);
     O.qwork = at<uint32_t>(geom, g.qwork);
+    O.sm = StagedMasks{at<uint64_t>(binning, bl.smask), at<uint64_t>(geom, g.stail)};
+    O.meta = meta;
+    O.sm_off = (uint32_t)(bl.smask / 256);
     const uint32_t* clist = at<const uint32_t>(binning, bl.clist);
     const float4* recs = at<const float4>(geom, g.rec);
     if (mode == BLEND_SPLIT) {
@@ -4312,6 +4396,9 @@ int render_backward_impl(bool full, int P, int64_t R, int W, int H, const float*
         const uint2* rng = at<uint2>(img, il.ranges);
         const uint32_t* clist = at<const uint32_t>(binning, bl.clist);
         const float4* recs = at<const float4>(geom, g.rec);
+        uint64_t* stail = at<uint64_t>(geom, g.stail);
+        char* bin = at<char>(const_cast<void*>(binning), 0);
+        const uint32_t* meta = at<const uint32_t>(geom, g.meta);
         // the split path's waves heaviest first (the forward recorded each
         // quadrant's work): the order is computed by eight blocks of the
         // kernel that clears the listed Gaussians' accumulators (every
@@ -4322,27 +4409,27 @@ int render_backward_impl(bool full, int P, int64_t R, int W, int H, const float*
         const unsigned zb = std::min<unsigned>(gs_div_up(4 * (size_t)P, 1024), 512u) + nsched;
         GS_TIMED("zero_gacc_kernel", stream,
                  hipLaunchKernelGGL(zero_gacc_kernel, dim3(zb), dim3(1024), 0, stream,
-                                    at<const uint32_t>(geom, g.meta), gacc, nsched, gx, gy, sgx, NS,
-                                    at<const uint32_t>(geom, g.qwork), sched, scnt));
+                                    meta, gacc, nsched, gx, gy, sgx, NS, at<const uint32_t>(geom, g.qwork), sched,
+                                    scnt));
         GS_LAUNCH_CHECK("zero_gacc_kernel");
         if (full) {
             GS_TIMED("render_bwd_kernel", stream,
                      hipLaunchKernelGGL(render_bwd_kernel<true>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
                                         NS, rng, clist, recs, compute_locally, bg, at<float>(img, il.final_T),
                                         at<uint32_t>(img, il.n_contrib), dL_dpixels, reinterpret_cast<float*>(gacc),
-                                        GeoBwd{}, nullptr, nullptr, ClearBuf{nullptr, 0}));
+                                        GeoBwd{}, nullptr, nullptr, stail, bin, meta, ClearBuf{nullptr, 0}));
         } else if (geo != nullptr) {
             GS_TIMED("render_bwd_geo_kernel", stream,
                      hipLaunchKernelGGL((render_bwd_kernel<false, true>), dim3(nblk), dim3(64), 0, stream, W, H, gx,
                                         gy, sgx, NS, rng, clist, recs, compute_locally, bg,
                                         at<float>(img, il.final_T), at<uint32_t>(img, il.n_contrib), dL_dpixels,
-                                        reinterpret_cast<float*>(gacc), *geo, sched, scnt, clr));
+                                        reinterpret_cast<float*>(gacc), *geo, sched, scnt, stail, bin, meta, clr));
         } else {
             GS_TIMED("render_bwd_kernel", stream,
                      hipLaunchKernelGGL(render_bwd_kernel<false>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
                                         NS, rng, clist, recs, compute_locally, bg, at<float>(img, il.final_T),
                                         at<uint32_t>(img, il.n_contrib), dL_dpixels, reinterpret_cast<float*>(gacc),
-                                        GeoBwd{}, sched, scnt, clr));
+                                        GeoBwd{}, sched, scnt, stail, bin, meta, clr));
         }
         GS_LAUNCH_CHECK("render_bwd_kernel");
     } else if (clr.n16 != 0) {
