@@ -6,7 +6,7 @@
 // reference's pruning is conservative, so its output is the exact 3-NN
 // statistic; it scans every box for every point (O(P^2/1024) box tests).
 //
-// Here: a uniform grid of about three points per cell is built with a counting
+// Here: a uniform grid of about 4.5 points per cell is built with a counting
 // sort (bbox reduce, cell histogram, device-wide scan, scatter), and every
 // point searches the cell shells around its own cell until the third-best
 // squared distance is below the distance to the unsearched region (computed
@@ -29,11 +29,12 @@ namespace {
 
 constexpr int RED_BLOCKS = 1024;
 constexpr int SCAN_BLOCK = 1024;
+constexpr int QT = 64;         // queries per block: one wave, whose LDS is free as soon as it ends
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct KnnLayout {
-    size_t partial, cell_of, count, start, blocksum, sorted, total;
+    size_t partial, cell_of, rank, count, start, blocksum, sorted, total;
 };
 
 // upper bound on the grid's cell count (the host grid rule enlarges the cell
@@ -47,6 +48,7 @@ constexpr KnnLayout knn_layout(int P)
     size_t o = 0;
     l.partial = o; o = align256(o + sizeof(float) * 6 * RED_BLOCKS);
     l.cell_of = o; o = align256(o + sizeof(uint32_t) * (size_t)P);
+    l.rank = o; o = align256(o + sizeof(uint32_t) * (size_t)P);
     l.count = o; o = align256(o + sizeof(uint32_t) * (NCmax + 1));
     l.start = o; o = align256(o + sizeof(uint32_t) * (NCmax + 1));
     l.blocksum = o; o = align256(o + sizeof(uint32_t) * ((NCmax + 1) / SCAN_BLOCK + 2));
@@ -88,6 +90,7 @@ __global__ __launch_bounds__(256) void bbox_partial_kernel(int P, const float* _
 
 struct Grid {
     double mn[3], hk[3];
+    double slack[3];   // bounds the rounding of cell coordinates and cell faces
     int n[3];
 };
 
@@ -103,7 +106,8 @@ __global__ __launch_bounds__(256) void zero_u32_kernel(size_t n, uint32_t* __res
 }
 
 __global__ __launch_bounds__(256) void cell_hist_kernel(int P, const float* __restrict__ pts, Grid g,
-                                                        uint32_t* __restrict__ cell_of, uint32_t* __restrict__ count)
+                                                        uint32_t* __restrict__ cell_of, uint32_t* __restrict__ rank,
+                                                        uint32_t* __restrict__ count)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P) return;
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256) void cell_hist_kernel(int P, const float* __re
     const int cz = cell_coord(pts[3 * (size_t)i + 2], g.mn[2], g.hk[2], g.n[2]);
     const uint32_t c = (uint32_t)((cz * g.n[1] + cy) * g.n[0] + cx);
     cell_of[i] = c;
-    atomicAdd(&count[c], 1u);
+    rank[i] = atomicAdd(&count[c], 1u);
 }
 
 // device-wide exclusive scan, three kernels: block scan + block sums, scan of
@@ -178,11 +182,13 @@ __global__ __launch_bounds__(256) void scan_add_kernel(size_t n, uint32_t* __res
 
 __global__ __launch_bounds__(256) void cell_scatter_kernel(int P, const float* __restrict__ pts,
                                                            const uint32_t* __restrict__ cell_of,
-                                                           uint32_t* __restrict__ cursor, float4* __restrict__ sorted)
+                                                           const uint32_t* __restrict__ rank,
+                                                           const uint32_t* __restrict__ start,
+                                                           float4* __restrict__ sorted)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P) return;
-    const uint32_t pos = atomicAdd(&cursor[cell_of[i]], 1u);
+    const uint32_t pos = start[cell_of[i]] + rank[i];
     sorted[pos] = make_float4(pts[3 * (size_t)i], pts[3 * (size_t)i + 1], pts[3 * (size_t)i + 2], __uint_as_float((uint32_t)i));
 }
 
@@ -200,28 +206,36 @@ __device__ __forceinline__ void upd3(float& b0, float& b1, float& b2, float d)
 }
 
 // candidates sorted[lo, hi) against the query at sorted position `self`; four
-// loads in flight
+// loads in flight, the last four clamped to the segment and masked
+__device__ __forceinline__ void scan_four(uint32_t k, uint32_t hi, const float4* __restrict__ sorted, float4 q,
+                                          uint32_t self, float& b0, float& b1, float& b2)
+{
+    float4 o[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) o[u] = sorted[min(k + u, hi - 1)];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) {
+        const float dx = o[u].x - q.x, dy = o[u].y - q.y, dz = o[u].z - q.z;
+        const float d = (dx * dx + dy * dy) + dz * dz;
+        upd3(b0, b1, b2, k + u >= hi || k + u == self ? __builtin_huge_valf() : d);
+    }
+}
+
 __device__ __forceinline__ void scan_segment(uint32_t lo, uint32_t hi, const float4* __restrict__ sorted, float4 q,
                                              uint32_t self, float& b0, float& b1, float& b2)
 {
-    uint32_t k = lo;
-    for (; k + 4 <= hi; k += 4) {
-        float4 o[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) o[u] = sorted[k + u];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const float dx = o[u].x - q.x, dy = o[u].y - q.y, dz = o[u].z - q.z;
-            const float d = (dx * dx + dy * dy) + dz * dz;
-            upd3(b0, b1, b2, k + u == self ? __builtin_huge_valf() : d);
-        }
-    }
-    for (; k < hi; k++) {
-        const float4 o = sorted[k];
-        const float dx = o.x - q.x, dy = o.y - q.y, dz = o.z - q.z;
-        const float d = (dx * dx + dy * dy) + dz * dz;
-        upd3(b0, b1, b2, k == self ? __builtin_huge_valf() : d);
-    }
+    for (uint32_t k = lo; k < hi; k += 4) scan_four(k, hi, sorted, q, self, b0, b1, b2);
+}
+
+// What a point `gap` cells beyond the neighbouring cell keeps from the query
+// along one axis, squared: `near` is the query's distance to that neighbour's
+// face.  The slack covers the double rounding of the cell coordinates and of the
+// faces, the relative margin the fp32 rounding of the distances it is compared
+// with (below 4e-7) and of this value.
+__device__ __forceinline__ float axis_gap2(double near, double h, int gap, double slack)
+{
+    const double d = fmax(near + (double)gap * h - slack, 0.0);
+    return (float)(d * d * (1.0 - 2e-6));
 }
 
 // distance from the query to the outside of the cell box c +- r (grid borders
@@ -233,8 +247,8 @@ __device__ __forceinline__ double box_bound(const Grid& g, const int (&c)[3], co
     for (int k = 0; k < 3; k++) {
         const double lo = g.mn[k] + (double)(c[k] - r) * g.hk[k];
         const double hi = g.mn[k] + (double)(c[k] + r + 1) * g.hk[k];
-        if (c[k] - r > 0) bound = fmin(bound, (double)qv[k] - lo);
-        if (c[k] + r + 1 < g.n[k]) bound = fmin(bound, hi - (double)qv[k]);
+        if (c[k] - r > 0) bound = fmin(bound, (double)qv[k] - lo - g.slack[k]);
+        if (c[k] + r + 1 < g.n[k]) bound = fmin(bound, hi - (double)qv[k] - g.slack[k]);
     }
     return bound;
 }
@@ -251,59 +265,117 @@ __device__ __forceinline__ bool box_done(double bound, float b2)
 // Queries run in cell order (one thread per sorted point), so a wave's
 // queries sit in neighbouring cells.  The 3x3x3 cells around the query are 9
 // runs of x-consecutive cells, i.e. 9 contiguous ranges of the cell-sorted
-// points; they are scanned first.  Only if the third-best distance is not yet
-// provably final are further shells visited cell by cell.
-__global__ __launch_bounds__(256) void knn_query_kernel(int P, Grid g, const uint32_t* __restrict__ start,
-                                                        const float4* __restrict__ sorted, float* __restrict__ out)
+// points.  The query's own run is scanned first; of the other eight a lane
+// keeps, in an LDS list, only the cells whose nearest face is not beyond its
+// third-best distance, and walks its list candidate by candidate.  Where the
+// points are denser than the grid's average that leaves about a quarter of the
+// candidates, and one flat loop over them costs a wave its longest lane's
+// total, not the sum over the runs of the longest lane in each.  Only if the
+// third-best distance is not yet provably final are further shells visited,
+// again without the rows that lie beyond it.  Bound by the latency of the
+// gathered candidates and by the longest lane of a wave.  10M points of a ground
+// plane with dense clusters: 4.96 ms with every run scanned in turn (3 points per
+// cell), 3.45 ms so at the same cells.
+__global__ __launch_bounds__(QT) void knn_query_kernel(int P, Grid g, const uint32_t* __restrict__ start,
+                                                       const float4* __restrict__ sorted, float* __restrict__ out)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint32_t s_lo[8][QT], s_hi[8][QT];
+    __shared__ float s_gap[8][QT];
+    const int t = threadIdx.x;
+    const int s = blockIdx.x * QT + t;
     if (s >= P) return;
     const float4 q = sorted[s];
     const uint32_t self = (uint32_t)s;   // the query's own position in the sorted points
     const float qv[3] = {q.x, q.y, q.z};
     int c[3];
+    double dlo[3], dhi[3];               // distances to the faces of the query's cell
 #pragma unroll
-    for (int k = 0; k < 3; k++) c[k] = cell_coord(qv[k], g.mn[k], g.hk[k], g.n[k]);
+    for (int k = 0; k < 3; k++) {
+        c[k] = cell_coord(qv[k], g.mn[k], g.hk[k], g.n[k]);
+        dlo[k] = (double)qv[k] - (g.mn[k] + (double)c[k] * g.hk[k]);
+        dhi[k] = (g.mn[k] + (double)(c[k] + 1) * g.hk[k]) - (double)qv[k];
+    }
     float b0 = FLT_MAX, b1 = FLT_MAX, b2 = FLT_MAX;
 
-    // r <= 1: nine row segments
+    // r <= 1
     {
         const int x0 = max(0, c[0] - 1), x1 = min(g.n[0] - 1, c[0] + 1);
-        uint32_t lo[9], hi[9];
+        const uint32_t own = (uint32_t)((c[2] * g.n[1] + c[1]) * g.n[0]);
+        scan_segment(start[own + (uint32_t)x0], start[own + (uint32_t)x1 + 1], sorted, q, self, b0, b1, b2);
+        float lo2[3], hi2[3];
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-            const int z = c[2] + j / 3 - 1, y = c[1] + j % 3 - 1;
+        for (int k = 0; k < 3; k++) {
+            lo2[k] = axis_gap2(dlo[k], g.hk[k], 0, g.slack[k]);
+            hi2[k] = axis_gap2(dhi[k], g.hk[k], 0, g.slack[k]);
+        }
+        // the four runs that share a face with the query's own come first
+        constexpr int DY[8] = {-1, 1, 0, 0, -1, 1, -1, 1}, DZ[8] = {0, 0, -1, 1, -1, -1, 1, 1};
+        uint32_t lo[8], hi[8];
+        float gap[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int z = c[2] + DZ[j], y = c[1] + DY[j];
+            gap[j] = (DY[j] < 0 ? lo2[1] : DY[j] > 0 ? hi2[1] : 0.f) + (DZ[j] < 0 ? lo2[2] : DZ[j] > 0 ? hi2[2] : 0.f);
             lo[j] = hi[j] = 0;
-            if (z >= 0 && z < g.n[2] && y >= 0 && y < g.n[1]) {
+            if (z >= 0 && z < g.n[2] && y >= 0 && y < g.n[1] && !(b2 < gap[j])) {
                 const uint32_t row = (uint32_t)((z * g.n[1] + y) * g.n[0]);
-                lo[j] = start[row + (uint32_t)x0];
-                hi[j] = start[row + (uint32_t)x1 + 1];
+                const int xa = b2 < gap[j] + lo2[0] ? c[0] : x0, xb = b2 < gap[j] + hi2[0] ? c[0] : x1;
+                lo[j] = start[row + (uint32_t)xa];
+                hi[j] = start[row + (uint32_t)xb + 1];
             }
         }
+        int n = 0;
 #pragma unroll
-        for (int j = 0; j < 9; j++) scan_segment(lo[j], hi[j], sorted, q, self, b0, b1, b2);
+        for (int j = 0; j < 8; j++) {
+            if (lo[j] < hi[j]) {
+                s_lo[n][t] = lo[j];
+                s_hi[n][t] = hi[j];
+                s_gap[n][t] = gap[j];
+                n++;
+            }
+        }
+        // a lane reads only what it wrote itself: no barrier
+        uint32_t k = 0, e = 0;
+        for (int i = 0;;) {
+            while (k >= e && i < n) {
+                k = s_lo[i][t];
+                e = b2 < s_gap[i][t] ? k : s_hi[i][t];
+                i++;
+            }
+            if (k >= e) break;
+            scan_four(k, e, sorted, q, self, b0, b1, b2);
+            k += 4;
+        }
     }
     const int rmax = max(g.n[0], max(g.n[1], g.n[2]));
     if (!box_done(box_bound(g, c, qv, 1), b2)) {
         for (int r = 2; r <= rmax; r++) {
             const int z0 = max(0, c[2] - r), z1 = min(g.n[2] - 1, c[2] + r);
             const int y0 = max(0, c[1] - r), y1 = min(g.n[1] - 1, c[1] + r);
+            const int xa = max(0, c[0] - r), xb = min(g.n[0] - 1, c[0] + r);
+            const float xlo2 = axis_gap2(dlo[0], g.hk[0], r - 1, g.slack[0]);
+            const float xhi2 = axis_gap2(dhi[0], g.hk[0], r - 1, g.slack[0]);
             for (int z = z0; z <= z1; z++) {
+                const float gz = z < c[2] ? axis_gap2(dlo[2], g.hk[2], c[2] - z - 1, g.slack[2])
+                               : z > c[2] ? axis_gap2(dhi[2], g.hk[2], z - c[2] - 1, g.slack[2]) : 0.f;
+                if (b2 < gz) continue;
                 for (int y = y0; y <= y1; y++) {
+                    const float gy = gz + (y < c[1] ? axis_gap2(dlo[1], g.hk[1], c[1] - y - 1, g.slack[1])
+                                         : y > c[1] ? axis_gap2(dhi[1], g.hk[1], y - c[1] - 1, g.slack[1]) : 0.f);
+                    if (b2 < gy) continue;
                     const uint32_t row = (uint32_t)((z * g.n[1] + y) * g.n[0]);
                     const bool shell_zy = (z == c[2] - r || z == c[2] + r || y == c[1] - r || y == c[1] + r);
                     if (shell_zy) {
                         // the whole x run of this shell row is new: one segment
-                        const int xa = max(0, c[0] - r), xb = min(g.n[0] - 1, c[0] + r);
                         scan_segment(start[row + (uint32_t)xa], start[row + (uint32_t)xb + 1], sorted, q, self, b0,
                                      b1, b2);
                     } else {
                         // interior rows: only the two x ends are new
-                        if (c[0] - r >= 0) {
+                        if (c[0] - r >= 0 && !(b2 < gy + xlo2)) {
                             const uint32_t cc = row + (uint32_t)(c[0] - r);
                             scan_segment(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
                         }
-                        if (c[0] + r < g.n[0]) {
+                        if (c[0] + r < g.n[0] && !(b2 < gy + xhi2)) {
                             const uint32_t cc = row + (uint32_t)(c[0] + r);
                             scan_segment(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
                         }
@@ -335,6 +407,7 @@ int knn_impl(int P, const float* points, float* out, void* workspace, hipStream_
     uint32_t* start = at<uint32_t>(workspace, L.start);
     uint32_t* bsum = at<uint32_t>(workspace, L.blocksum);
     float4* sorted = at<float4>(workspace, L.sorted);
+    uint32_t* rank = at<uint32_t>(workspace, L.rank);   // a point's place in its cell
 
     const int nred = (int)std::min<size_t>(RED_BLOCKS, gs_div_up((size_t)P, 256));
     GS_TIMED("knn_bbox_kernel", stream,
@@ -358,10 +431,13 @@ int knn_impl(int P, const float* points, float* out, void* workspace, hipStream_
         if (ext[k] < 1e-12) ext[k] = 1e-12;
         vol *= ext[k];
     }
-    // about three points per cell (measured: 2 -> 3 per cell is -11 % on a ground
-    // plane with dense clusters, -3.5 % on uniform points; 1 or >= 4 are slower),
+    // about 4.5 points per cell: coarser cells spare the points in the sparse parts
+    // their shells, and the query skips what they add elsewhere (measured, whole
+    // call, at 2 / 3 / 4.5 / 6 / 8 per cell: 10M points of a ground plane with dense
+    // clusters 4.82 / 3.97 / 3.61 / 3.62 / 3.78 ms, 100k in clusters
+    // 157 / 133 / 136 / 162 / 165 us, 1M uniform 204 / 208 / 205 / 209 / 205 us),
     // at most 1024 cells per axis and max_cells(P) in total
-    double h = cbrt(vol / ((double)P / 3.0 + 1.0));
+    double h = cbrt(vol / ((double)P / 4.5 + 1.0));
     size_t NC = 0;
     for (int iter = 0; iter < 200; iter++) {
         NC = 1;
@@ -379,13 +455,14 @@ int knn_impl(int P, const float* points, float* out, void* workspace, hipStream_
     for (int k = 0; k < 3; k++) {
         g.mn[k] = mn[k];
         g.hk[k] = ext[k] / g.n[k];
+        g.slack[k] = 4e-15 * (std::fabs(mn[k]) + ext[k]);
     }
     GS_TIMED("knn_zero_kernel", stream,
              hipLaunchKernelGGL(zero_u32_kernel, dim3(1024), dim3(256), 0, stream, NC + 1, count));
     GS_LAUNCH_CHECK("zero_u32_kernel");
     GS_TIMED("knn_hist_kernel", stream,
              hipLaunchKernelGGL(cell_hist_kernel, dim3(gs_div_up((size_t)P, 256)), dim3(256), 0, stream, P, points, g,
-                                cell_of, count));
+                                cell_of, rank, count));
     GS_LAUNCH_CHECK("cell_hist_kernel");
     const size_t n = NC + 1;
     const unsigned nb = gs_div_up(n, SCAN_BLOCK);
@@ -398,14 +475,12 @@ int knn_impl(int P, const float* points, float* out, void* workspace, hipStream_
     GS_TIMED("knn_scan_add_kernel", stream,
              hipLaunchKernelGGL(scan_add_kernel, dim3(gs_div_up(n, 256)), dim3(256), 0, stream, n, start, bsum));
     GS_LAUNCH_CHECK("scan_add_kernel");
-    // cursor = copy of start (reuse `count`)
-    GS_HIP(hipMemcpyAsync(count, start, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, stream));
     GS_TIMED("knn_scatter_kernel", stream,
              hipLaunchKernelGGL(cell_scatter_kernel, dim3(gs_div_up((size_t)P, 256)), dim3(256), 0, stream, P, points,
-                                cell_of, count, sorted));
+                                cell_of, rank, start, sorted));
     GS_LAUNCH_CHECK("cell_scatter_kernel");
     GS_TIMED("knn_query_kernel", stream,
-             hipLaunchKernelGGL(knn_query_kernel, dim3(gs_div_up((size_t)P, 256)), dim3(256), 0, stream, P, g, start,
+             hipLaunchKernelGGL(knn_query_kernel, dim3(gs_div_up((size_t)P, QT)), dim3(QT), 0, stream, P, g, start,
                                 sorted, out));
     GS_LAUNCH_CHECK("knn_query_kernel");
     GS_HIP(hipStreamSynchronize(stream));
@@ -430,7 +505,7 @@ extern "C" int gs_knn_meandist3(int P, const float* points, float* out, void* wo
 // allocate (serving loops, harnesses that forbid hipMalloc).  It cannot be
 // captured into a HIP graph: like gs_knn_meandist3 it reads the bounding box
 // back to the host mid-call and synchronises the stream.  Each GPU the library
-// runs on holds its own copy of the array (KNN_SCRATCH_BYTES, about 38 MB)
+// runs on holds its own copy of the array (KNN_SCRATCH_BYTES, about 42 MB)
 // until the process ends.  In host code `scratch` names a host-side stand-in,
 // never the device memory: the per-device address comes from
 // hipGetSymbolAddress on the first call on each device and only that address

@@ -340,7 +340,7 @@ int gs_knn_meandist3(int P, const float* points, float* out, void* workspace, gs
 /* Allocation-free distCUDA2.  No counterpart in the reference: for callers
  * that cannot allocate device memory (tight serving loops, harnesses that
  * forbid hipMalloc).  Same result as gs_knn_meandist3, with the workspace in
- * a device array inside the library (about 38 MB, held on every GPU the
+ * a device array inside the library (about 42 MB, held on every GPU the
  * library runs on until the process ends) instead of a caller buffer;
  * allocates nothing.  Not for HIP graph capture: it reads the points'
  * bounding box back to the host mid-call and synchronises `stream`.

@@ -37,6 +37,30 @@ def test_knn_bitexact(n, kind):
     assert_bitexact(got, ref, f"distCUDA2 {kind} n={n}")
 
 
+@pytest.mark.parametrize("kind", ["lattice", "one_cluster", "offset", "line", "pairs"])
+@pytest.mark.parametrize("n", [63, 4097, 30011])
+def test_knn_skipped_rows_bitexact(n, kind):
+    # points whose neighbours lie in skipped or trimmed rows if a bound is too
+    # tight: ties on cell faces, dense and empty cells side by side, coordinates
+    # far from zero, single-cell axes, near-duplicates across the grid
+    from blitzgs_amd.knn import distCUDA2
+    rng = np.random.default_rng(n)
+    if kind == "lattice":
+        k = int(np.ceil(n ** (1 / 3)))
+        pts = np.stack(np.meshgrid(*[np.arange(k)] * 3), -1).reshape(-1, 3)[:n] * 0.25
+    elif kind == "one_cluster":
+        pts = np.concatenate([rng.normal(0, 0.01, (n - n // 50, 3)), rng.uniform(-10, 10, (n // 50, 3))])
+    elif kind == "offset":
+        pts = rng.uniform(0, 1, (n, 3)) + np.array([1000.0, -3000.0, 7.0])
+    elif kind == "line":
+        pts = np.concatenate([rng.uniform(-5, 5, (n, 1)), np.zeros((n, 2))], 1)
+    else:
+        half = rng.uniform(-1, 1, ((n + 1) // 2, 3))
+        pts = np.concatenate([half, half + rng.normal(0, 1e-7, half.shape)])[:n]
+    pts = np.ascontiguousarray(pts, np.float32)
+    assert_bitexact(np_(distCUDA2(to_dev(pts))), O.knn_meandist3(pts), f"distCUDA2 {kind} n={n}")
+
+
 def test_knn_dropin_module():
     import sys, os
     sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(__file__)), "blitzgs_amd", "dropin"))
