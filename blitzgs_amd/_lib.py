@@ -73,6 +73,9 @@ _SIGS = {
     "gs_knn_meandist3_noalloc": (_i, [_i, _c, _c, _c]),
     "gs_ssim_forward": (_i, [_i, _i, _i, _i, _f, _f, _c, _c, _c, _c, _c, _c, _c]),
     "gs_ssim_backward": (_i, [_i, _i, _i, _i, _f, _f, _c, _c, _c, _c, _c, _c, _c, _c]),
+    "gs_ssim_mean_workspace_bytes": (_sz, [_i, _i, _i, _i]),
+    "gs_ssim_mean_forward": (_i, [_i, _i, _i, _i, _f, _f, _c, _c, _i, _c, _c, _c, _c, _c, _c]),
+    "gs_ssim_mean_backward": (_i, [_i, _i, _i, _i, _c, _c, _i, _c, _c, _c, _c, _c, _c]),
     "gs_adam_update": (_i, [_c, _c, _c, _c, _c, _f, _f, _f, _f, _i64, _i64, _c]),
     "gs_adam_update_groups": (_i, [_i, C.POINTER(AdamGroup), _i64, _c, _f, _f, _c]),
     "gs_preprocess_forward_full": (_i, [_i, _i, _i, _c, _c, _c, _c, _c, _c, _c, _c, _c, _f, _c, _c, _c, _f, _f, _i,

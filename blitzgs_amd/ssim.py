@@ -94,8 +94,53 @@ class FusedSSIMMap(torch.autograd.Function):
         return None, None, dL_dimg1, None, None, None
 
 
+class FusedSSIMMean(torch.autograd.Function):
+    """The mean of the SSIM map (without its 5-pixel border for "valid") as one
+    node: the map is not stored, and the backward takes dL/dmean as it is."""
+
+    @staticmethod
+    def forward(ctx, C1, C2, img1, img2, border, train):
+        a = img1.detach().to(torch.float32).contiguous()
+        b = img2.to(torch.float32).contiguous()
+        B, Ch, H, W = a.shape
+        lib = _lib.load()
+        mean = torch.empty((), device=a.device, dtype=torch.float32)
+        ws = torch.empty(lib.gs_ssim_mean_workspace_bytes(B, Ch, H, W), device=a.device, dtype=torch.uint8)
+        partials = [torch.empty_like(a) if train else torch.empty(0, device=a.device) for _ in range(3)]
+        p = [_lib.ptr(t) if train else None for t in partials]
+        _lib.check(lib.gs_ssim_mean_forward(B, Ch, H, W, float(C1), float(C2), _lib.ptr(a), _lib.ptr(b), border,
+                                            _lib.ptr(mean), _lib.ptr(ws), *p, _stream(a.device)),
+                   "gs_ssim_mean_forward")
+        ctx.border = border
+        ctx.save_for_backward(img1.detach(), img2, *partials)
+        return mean
+
+    @staticmethod
+    def backward(ctx, grad_mean):
+        img1, img2, *partials = ctx.saved_tensors
+        a = img1.to(torch.float32).contiguous()
+        b = img2.to(torch.float32).contiguous()
+        B, Ch, H, W = a.shape
+        dL = grad_mean.to(torch.float32).contiguous()
+        partials = [t.contiguous() for t in partials]
+        g = torch.empty_like(a)
+        _lib.check(_lib.load().gs_ssim_mean_backward(B, Ch, H, W, _lib.ptr(a), _lib.ptr(b), ctx.border, _lib.ptr(dL),
+                                                     *(_lib.ptr(t) for t in partials), _lib.ptr(g),
+                                                     _stream(a.device)),
+                   "gs_ssim_mean_backward")
+        return None, None, g, None, None, None
+
+
 def fused_ssim(img1, img2, padding="same", train=True):
     """Mean SSIM of img1 against img2 (fused_ssim/__init__.py:37-41)."""
     if padding not in allowed_padding:
         raise AssertionError(f"padding must be one of {allowed_padding}, got {padding!r}")
-    return FusedSSIMMap.apply(_SSIM_C1, _SSIM_C2, img1, img2, padding, train).mean()
+    _check_img(img1, "img1")
+    _check_img(img2, "img2")
+    if img1.shape != img2.shape:
+        raise RuntimeError("img1 and img2 must have the same shape")
+    border = _BORDER if padding == "valid" else 0
+    if img1.numel() == 0 or min(img1.shape[-2:]) <= 2 * border:
+        # the mean over no pixel, and its gradient, are torch's
+        return FusedSSIMMap.apply(_SSIM_C1, _SSIM_C2, img1, img2, padding, train).mean()
+    return FusedSSIMMean.apply(_SSIM_C1, _SSIM_C2, img1, img2, border, train)

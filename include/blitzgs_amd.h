@@ -364,6 +364,17 @@ int gs_ssim_backward(int B, int C, int H, int W, float C1, float C2, const float
                      const float* dm_dsigma1_sq, const float* dm_dsigma12, float* dL_dimg1,
                      gs_stream_t stream);
 
+/* The loss's form of the two: the mean of the map without `border` pixels on
+ * every side (H and W > 2 border), and dL/dimg1 from the one device value
+ * dL_dmean.  The workspace is only needed during the forward. */
+size_t gs_ssim_mean_workspace_bytes(int B, int C, int H, int W);
+int gs_ssim_mean_forward(int B, int C, int H, int W, float C1, float C2, const float* img1,
+                         const float* img2, int border, float* mean, void* workspace, float* dm_dmu1,
+                         float* dm_dsigma1_sq, float* dm_dsigma12, gs_stream_t stream);
+int gs_ssim_mean_backward(int B, int C, int H, int W, const float* img1, const float* img2, int border,
+                          const float* dL_dmean, const float* dm_dmu1, const float* dm_dsigma1_sq,
+                          const float* dm_dsigma12, float* dL_dimg1, gs_stream_t stream);
+
 /* ------------------------------------------------------------------------ *
  * Sparse Adam step.  gs_adam_update replaces the reference's adamUpdate
  * (diff-gaussian-rasterization_f/rasterize_points.cu:807-832, kernel

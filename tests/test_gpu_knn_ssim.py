@@ -87,6 +87,27 @@ def test_ssim_forward_backward_bitexact(shape):
     assert_bitexact(np_(m2), om, "ssim_map (train=False)")
 
 
+@pytest.mark.parametrize("padding", ["same", "valid"])
+@pytest.mark.parametrize("shape", [(1, 1, 11, 11), (1, 3, 64, 256), (2, 1, 65, 257), (3, 2, 139, 300)])
+def test_fused_ssim_mean_against_map(shape, padding):
+    # the one-node mean against the map's own path: the gradient has the same
+    # operations (bit-exact); the mean differs from the fp64 mean of the map by
+    # its rounding to fp32 alone (half an ulp; the fp64 sums add far less)
+    from blitzgs_amd.ssim import FusedSSIMMap, fused_ssim
+    rng = np.random.default_rng(sum(shape))
+    x, y = (rng.random(shape).astype(np.float32) for _ in range(2))
+    xa, xb = to_dev(x).requires_grad_(True), to_dev(x).requires_grad_(True)
+    m = FusedSSIMMap.apply(0.01 ** 2, 0.03 ** 2, xa, to_dev(y), padding, True)
+    v = fused_ssim(xb, to_dev(y), padding)
+    ref = float(m.detach().double().mean())
+    assert abs(float(v.detach()) - ref) <= 2 ** -23 * abs(ref)
+    (3.0 * m.mean()).backward()
+    (3.0 * v).backward()
+    assert_bitexact(np_(xb.grad), np_(xa.grad), "dL_dimg1")
+    with torch.no_grad():
+        assert float(fused_ssim(to_dev(x), to_dev(y), padding, False)) == float(v.detach())
+
+
 def test_fused_ssim_autograd_same_and_valid():
     import sys, os
     sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(__file__)), "blitzgs_amd", "dropin"))
