@@ -105,11 +105,6 @@ __device__ __forceinline__ float blend_g(float power, float cut_power)
     return G;
 }
 
-__device__ __forceinline__ float blend_opacity_g(float opacity, float power, float cut_power)
-{
-    return opacity * blend_g(power, cut_power);
-}
-
 // alpha = min(0.99, opacity * G); G is returned too
 __device__ __forceinline__ float blend_alpha(float opacity, float power, float cut_power, float& G)
 {

@@ -3260,7 +3260,8 @@ struct BwdConst {
 // updates the pixel's state and yields the entry's gradient factors.
 struct BwdEval {
     float dy, hadx, hcdy, nbdx;
-    float oG;   // opacity G, 0 where the pixel does not blend the entry
+    float G, alpha;   // 0 where the pixel does not blend the entry
+    bool clamped;     // the alpha clamp is active
     bool valid;
 };
 
@@ -3277,9 +3278,12 @@ __device__ __forceinline__ BwdEval bwd_eval(const BwdConst& k, const float4& A, 
     e.nbdx = A.w * dx;
     const float power = __builtin_fmaf(e.hadx, dx, __builtin_fmaf(e.hcdy, e.dy, e.nbdx * e.dy));
     // alpha = min(0.99, opacity G): its cut at 1/255 is opacity G's
-    const float oG = gs::blend_opacity_g(B.y, power, Cc.w);
+    const float G = gs::blend_g(power, Cc.w);
+    const float oG = B.y * G;
     e.valid = ci1 <= k.last && !(power > 0.0f) && !(oG < (1.0f / 255.0f));
-    e.oG = e.valid ? oG : 0.f;
+    e.clamped = oG > 0.99f;
+    e.G = e.valid ? G : 0.f;
+    e.alpha = e.valid ? __builtin_fminf(0.99f, oG) : 0.f;
     return e;
 }
 
@@ -3297,11 +3301,12 @@ __device__ __forceinline__ float swap16_add(float a, float b)
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// An entry's per-pixel gradient factors.  With w = dL/dG G, v = alpha T and
+// An entry's per-pixel gradient factors.  With w = dL/dalpha G, v = alpha T and
 // d = mean - pixel, every gradient term of the entry is a sum over the pixels
 // of w or v times a per-pixel constant, of |w dG/dmean| or (FULL) of the
-// unclamped w:  dmean = sum w (2 ha dx + nb dy, 2 hc dy + nb dx), dconic ~
-// sum w (dx dx, dx dy, dy dy), dopacity = sum w / opacity, drgb = sum v dL/dpixel.
+// unclamped w:  dmean = o sum w (2 ha dx + nb dy, 2 hc dy + nb dx), dconic ~
+// o sum w (dx dx, dx dy, dy dy), dopacity = sum w, drgb = sum v dL/dpixel, o the
+// opacity (applied to the sums: dopacity takes no division).
 struct BwdTerms {
     float w, v;
     float u;   // split: |w dpx| (lanes < 32) and |w dpy| (>= 32), each summed over lanes l and l ^ 32;
@@ -3310,20 +3315,20 @@ struct BwdTerms {
 
 // Branch-free: every lane applies the entry; a lane whose pixel does not
 // blend it (past its last contributor, power > 0, alpha < 1/255) gets zero
-// gradient factors and unchanged state through the one factor opacity G.  GEO (render_geo): m_dp is the entry's five
-// maps dotted with the pixel's map gradients; the maps join the colour in
-// every dot product (the accumulation is the same linear rule for all eight
-// channels).
+// gradient factors and unchanged state through its zero G and alpha.  GEO
+// (render_geo): m_dp is the entry's five maps dotted with the pixel's map
+// gradients; the maps join the colour in every dot product (the accumulation
+// is the same linear rule for all eight channels).
 template <bool FULL, bool GEO = false>
 __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, const float4& A, const float4& B,
                                               const float4& Cc, const BwdEval& e,
                                               [[maybe_unused]] float m_dp = 0.f)
 {
-    // a lane that does not blend the entry runs it with opacity G = alpha = 0:
-    // T and the colour behind it are unchanged (1 / (1 - 0) is exactly 1), and
-    // every gradient term carries a factor alpha (colour) or opacity G (the
-    // others; dL/dalpha stays finite)
-    const float alpha = __builtin_fminf(0.99f, e.oG);
+    // a lane that does not blend the entry runs it with G = alpha = 0: T and
+    // the colour behind it are unchanged (1 / (1 - 0) is exactly 1), and every
+    // gradient term carries a factor alpha (colour) or G (the others; dL/dalpha
+    // stays finite)
+    const float alpha = e.alpha;
     const float inv_one_m = __builtin_amdgcn_rcpf(1.f - alpha);   // 1 ulp; gradients only
     p.T = p.T * inv_one_m;
     BwdTerms t;
@@ -3339,9 +3344,9 @@ __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, co
     const float d_dp = e.valid ? c_dp - p.acc_dp : 0.f;   // (a colour that is not finite stays with the pixels it enters)
     p.acc_dp = __builtin_fmaf(alpha, d_dp, p.acc_dp);
     const float dL_dalpha = __builtin_fmaf(d_dp, p.T, inv_one_m * k.nT_bg);
-    const float w = dL_dalpha * e.oG;
+    const float w = dL_dalpha * e.G;
     if constexpr (FULL) {
-        t.w = e.oG > 0.99f ? 0.f : w;
+        t.w = e.clamped ? 0.f : w;
         t.u = w;
     } else {
         // dG/ddelx = G (2 ha dx + nb dy), dG/ddely = G (2 hc dy + nb dx)
@@ -3357,12 +3362,17 @@ __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, co
 //
 // Each blended entry leaves its rows w, v, u (64 pixels) in LDS; after four,
 // lane l takes entry (l >> 1) & 3 and four consecutive pixels of it, forms
-// the entry's eleven terms summed over those four (the w moments from sum w,
-// sum i w, sum i i w) and the terms are summed over the entry's sixteen lanes.
+// the entry's eleven terms summed over those four and the terms are summed
+// over the entry's sixteen lanes.  The offsets of the four pixels from the
+// mean are taken one by one (each exact where it is small): moments about one
+// of them (sum w, sum i w, sum i i w) are fewer instructions, but cancel where
+// a narrow Gaussian's weight sits on one pixel near its mean (up to half of a
+// faint one's conic sum was lost).
 //
 // Bound: the walk is bound by VALU issue.  Forming the eleven terms per pixel
-// and summing each over 64 lanes by transpose-adds took 36 VALU instructions
-// of an entry's 84; this takes 19 (and 5 for the rows).  Measured (render
+// and summing each over 64 lanes by transpose-adds made an entry 82 VALU
+// instructions; this makes it 60 (58 with the moments; counted on the probe).
+// Measured (render
 // backward, before -> after): 6M aerial Gaussians at 1600x1066 642 -> 510 us,
 // 1M wide ones at 1920x1080 367 -> 284 us, the full-image path's 2M at
 // 1237x822 377 -> 225 us.  Tried: the sums as a contraction on the matrix
@@ -3478,23 +3488,21 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
     const float4 A = st.a[j];
     const float2 B = *reinterpret_cast<const float2*>(&st.b[j]);
     const uint32_t cx = __float_as_uint(st.c[j].y);
-    const float dx = A.x - g.x0, dy = A.y - g.y;   // the first pixel's; the others' dx - 1, - 2, - 3
+    const float dx0 = A.x - g.x0, dx1 = dx0 - 1.f, dx2 = dx0 - 2.f, dx3 = dx0 - 3.f, dy = A.y - g.y;
     const float s = (w.x + w.y) + (w.z + w.w);
-    const float i1 = __builtin_fmaf(3.f, w.w, __builtin_fmaf(2.f, w.z, w.y));
-    const float i2 = __builtin_fmaf(9.f, w.w, __builtin_fmaf(4.f, w.z, w.y));
-    const float wx = __builtin_fmaf(dx, s, -i1), wy = dy * s;
-    const float wxx = __builtin_fmaf(dx, wx, __builtin_fmaf(-dx, i1, i2)), wxy = dy * wx, wyy = dy * wy;
+    const float wx0 = w.x * dx0, wx1 = w.y * dx1, wx2 = w.z * dx2, wx3 = w.w * dx3;
+    const float wx = (wx0 + wx1) + (wx2 + wx3), wy = dy * s;
+    const float wxx = __builtin_fmaf(wx3, dx3, __builtin_fmaf(wx2, dx2, __builtin_fmaf(wx1, dx1, wx0 * dx0)));
+    const float wxy = dy * wx, wyy = dy * wy;
     float fx = wx, fy = wy, p23;
     if constexpr (FULL) {
-        const float f = (u.x + u.y) + (u.z + u.w);
-        fx = __builtin_fmaf(dx, f, -__builtin_fmaf(3.f, u.w, __builtin_fmaf(2.f, u.z, u.y)));
-        fy = dy * f;
+        fx = __builtin_fmaf(u.w, dx3, __builtin_fmaf(u.z, dx2, __builtin_fmaf(u.y, dx1, u.x * dx0)));
+        fy = dy * ((u.x + u.y) + (u.z + u.w));
         p23 = 0.f;   // not read
     } else {
         p23 = (u.x + u.y) + (u.z + u.w);
     }
     const float gx = __builtin_fmaf(2.f * A.z, fx, A.w * fy), gy = __builtin_fmaf(2.f * B.x, fy, A.w * fx);
-    const float gop = s * __builtin_amdgcn_rcpf(B.y);
     auto dot = [&](const float (&d)[4]) {
         return __builtin_fmaf(v.w, d[3], __builtin_fmaf(v.z, d[2], __builtin_fmaf(v.y, d[1], v.x * d[0])));
     };
@@ -3507,10 +3515,10 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
     } else {
         pab = swap32_add(c2, c2);
     }
-    const float sum = grad_reduce<GEO>(swap32_add(gx, gy), p23, swap32_add(wxx, wxy), swap32_add(wyy, gop),
+    const float sum = grad_reduce<GEO>(swap32_add(gx, gy), p23, swap32_add(wxx, wxy), swap32_add(wyy, s),
                                        swap32_add(dot(g.dp[0]), dot(g.dp[1])), pab, pcd, pef, lane);
     lds_order();
-    return GradSum{sum, cx};
+    return GradSum{grad_slot(lane) < 7 ? B.y * sum : sum, cx};   // slots 0 .. 6: the mean's and the conic's
 }
 
 template <bool FULL, bool GEO>
