@@ -3472,8 +3472,8 @@ struct GradSum {
     uint32_t cx;   // of this accumulator row
 };
 
-// The sums of the four entries staged from j0 on.  grad_flush adds the first
-// n of them to the accumulators.
+// The sums of the four entries staged from j0 on.  grad_flush adds those whose
+// bit is set in `blended` to the accumulators.
 template <bool FULL, bool GEO>
 __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels<GEO>& g, const Stage& st,
                                              int j0, int lane)
@@ -3523,11 +3523,11 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
 
 template <bool FULL, bool GEO>
 __device__ __forceinline__ void grad_flush(const float* rows, const GradPixels<GEO>& g, const Stage& st,
-                                           int j0, int n, int lane, float* __restrict__ gacc)
+                                           int j0, uint32_t blended, int lane, float* __restrict__ gacc)
 {
     const GradSum t = grad_sums<FULL, GEO>(rows, g, st, j0, lane);
     const int i = grad_slot(lane);
-    const bool on = ((lane >> 1) & 3) < n && i < (GEO ? 16 : 11) && !(FULL && (i == 2 || i == 3));
+    const bool on = ((blended >> ((lane >> 1) & 3)) & 1u) != 0 && i < (GEO ? 16 : 11) && !(FULL && (i == 2 || i == 3));
     if (on) unsafeAtomicAdd(gacc + (size_t)t.cx * 16 + i, t.v);
 }
 
@@ -3755,6 +3755,12 @@ __device__ __forceinline__ void render_bwd_body(
         }
         __syncthreads();
         for (int j0 = 0; j0 < cnt; j0 += GRAD_SLOTS) {
+            // the entries of this group that a pixel blends: on the split path
+            // every marked one; on the full-image path, where the forward marks
+            // what it staged, those found here (an entry that no pixel blends
+            // takes no sum: a gradient that is not finite would make its zero
+            // factors NaN)
+            uint32_t blended = FULL ? 0u : (1u << min(cnt - j0, GRAD_SLOTS)) - 1u;
 #pragma unroll
             for (int s = 0; s < GRAD_SLOTS; s++) {
                 const int j = j0 + s;
@@ -3762,6 +3768,7 @@ __device__ __forceinline__ void render_bwd_body(
                 const float4 B = st.b[j];
                 const float4 Cc = st.c[j];
                 const BwdEval e = bwd_eval(kc, A, B, Cc);
+                if constexpr (FULL) blended |= gs::ballot(e.valid) != 0 ? 1u << s : 0u;
                 float m_dp = 0.f;
                 if constexpr (GEO) {
                     m_dp = st_map[j] * dm[0];
@@ -3769,7 +3776,8 @@ __device__ __forceinline__ void render_bwd_body(
                 }
                 grad_put(rows, s, lane, bwd_apply<FULL, GEO>(px_st, kc, A, B, Cc, e, m_dp));
             }
-            grad_flush<FULL, GEO>(rows, gp, st, j0, cnt - j0, lane, gacc);
+            if (FULL && blended == 0u) continue;
+            grad_flush<FULL, GEO>(rows, gp, st, j0, blended, lane, gacc);
         }
         __syncthreads();
     }

@@ -162,3 +162,36 @@ def test_narrow(gpu, path, seed, faint):
         bad = np.abs(g - ref[k]) > bound[k]
         i = np.unravel_index((np.abs(g - ref[k]) / np.maximum(bound[k], 1e-300)).argmax(), g.shape)
         assert int(bad.sum()) == 0, (k, int(bad.sum()), i, g[i], ref[k][i], bound[k][i])
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("n", [1, 4, 6, 70])
+def test_full_path_unblended_entries_take_no_gradient(gpu, n, value):
+    """Full-image path: faint Gaussians whose means lie between pixel centres
+    are staged (the test that drops entries is against the quadrant's rectangle)
+    and blended by no pixel.  Beside blended ones and with an image gradient that
+    is not finite in their quadrant they take no gradient, and the blended ones of
+    the other quadrants take what they take without it."""
+    rng = np.random.default_rng(n)
+    m = rng.integers(0, 6, (n, 2)) + 0.5
+    op = np.full(n, 1.2 / 255)
+    seen = np.arange(n) % 3 == 1     # these are blended, every other one in the quadrant at (8, 0)
+    op[seen] = 0.4
+    m[seen] += np.where(np.arange(int(seen.sum())) % 2 == 1, 8.0, 0.0)[:, None] * [[1.0, 0.0]] + 0.5
+    other = seen & (m[:, 0] > 8)
+    m[other] = [12.0, 4.0]
+    s = 1 / 0.3
+    x = dict(means2D=m.astype(np.float32), conic=np.stack([np.full(n, s), np.zeros(n), np.full(n, s), op], 1).astype(np.float32),
+             rgb=rng.uniform(0, 1, (n, 3)).astype(np.float32), radii=np.full(n, 4, np.int32),
+             depths=np.arange(n, dtype=np.float32) + 1, bg=np.zeros(3, np.float32),
+             dL=rng.standard_normal((3, H, W)).astype(np.float32))
+    x["conic"][other, 0] = x["conic"][other, 2] = 2.0   # within 8 .. 15
+    want = _full(x)
+    bad = x["dL"].copy()
+    bad[:, 2, 3] = value
+    got = _full(x, dL=bad)
+    for k in got:
+        a, b = np_(got[k]), np_(want[k])
+        assert not a[~seen].any() and not b[~seen].any(), k
+        # three additions in another order
+        assert (np.abs(a[other] - b[other]) <= 6e-7 * np.abs(b[other]).max(initial=0.0)).all(), k
