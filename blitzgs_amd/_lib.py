@@ -57,6 +57,8 @@ _SIGS = {
     "gs_render_forward": (_i, [_i, _i64, _i, _i, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c,
                                _c, _i, _c, _i64, _c]),
     "gs_render_forward_reserved": (_i, [_i, _i64, _i, _i] + [_c] * 15 + [C.POINTER(_i64), _i, _c, _i64, _c]),
+    "gs_render_view": (_i, [_i, _i64, _i, _i] + [_c] * 15 + [_i, _c, _i64, _c]),
+    "gs_render_view_reserved": (_i, [_i, _i64, _i, _i] + [_c] * 15 + [C.POINTER(_i64), _i, _c, _i64, _c]),
     "gs_render_backward": (_i, [_i, _i64, _i, _i, _c, _c, _c, _c, _c, _c, _c, _c, _c, _c, _i, _c, _c, _c, _c,
                                 _i64, _c]),
     "gs_render_geo_forward": (_i, [_i, _i64, _i, _i, _f, _f, _c, _c, _c, _c, _c, _c, _c, _c]),

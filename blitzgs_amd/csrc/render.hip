@@ -2605,8 +2605,17 @@ constexpr int BLEND_GEO = 4;
 // the split path's render and render_geo's maps in one walk: the colour
 // outputs and statistics of BLEND_SPLIT, the maps and plane depth of BLEND_GEO
 constexpr int BLEND_SPLIT_GEO = 5;
-__host__ __device__ constexpr bool is_split(int mode) { return mode == BLEND_SPLIT || mode == BLEND_SPLIT_GEO; }
+// BLEND_SPLIT for a view that no backward follows: no entry is marked, and the
+// pixels' contributor counts are left at zero, so that a backward over them
+// walks nothing.  Finding the marked entries and writing the marks is 5 % of
+// the blend: 192 -> 178 us at 1M wide Gaussians, 1920x1080; 66 -> 61 us at 16k, 256x256
+constexpr int BLEND_VIEW = 6;
+__host__ __device__ constexpr bool is_split(int mode)
+{
+    return mode == BLEND_SPLIT || mode == BLEND_SPLIT_GEO || mode == BLEND_VIEW;
+}
 __host__ __device__ constexpr bool is_geo(int mode) { return mode == BLEND_GEO || mode == BLEND_SPLIT_GEO; }
+__host__ __device__ constexpr bool has_marks(int mode) { return mode != BLEND_GEO && mode != BLEND_VIEW; }
 constexpr int NUM_MAPS = 5;   // NUM_ALL_MAP (_r config.h:24)
 
 // A caller's buffer that a blend kernel clears while it runs (n16: 16-byte
@@ -2685,8 +2694,8 @@ struct FwdOut {
     float* out_plane_depth;        // geo: (H,W)
     float focal_x, focal_y, cx, cy;   // geo: the plane depth's pixel rays
     ClearBuf clr;                  // split: a caller's buffer cleared after the walks (none: n16 == 0)
-    StagedMasks sm;                // all but BLEND_GEO
-    uint32_t* meta;                // ... which leaves sm.full's place in meta[11]
+    StagedMasks sm;                // has_marks
+    uint32_t* meta;                // ... whose launch leaves sm.full's place in meta[11]
     uint32_t sm_off;
 };
 
@@ -2699,7 +2708,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     const float* __restrict__ bg, FwdOut O)
 {
     [[maybe_unused]] const ClearAtExit clear_at_exit{O.clr};
-    if (MODE != BLEND_GEO && blockIdx.x == 0 && threadIdx.x == 0) O.meta[11] = O.sm_off;
+    if (has_marks(MODE) && blockIdx.x == 0 && threadIdx.x == 0) O.meta[11] = O.sm_off;
     unsigned tile, quad, tx, ty;
     if (!block_to_tile(blockIdx.x, gx, gy, sgx, NS, tile, quad, tx, ty)) return;
     const int lane = threadIdx.x;
@@ -2789,7 +2798,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
             const FwdStep f = fwd_blend_step(px_st, A, B, Cc, pxf, pyf);
             const bool upd = f.upd;
             const float wgt = f.wgt;
-            if constexpr (is_split(MODE)) {
+            if constexpr (is_split(MODE) && has_marks(MODE)) {
                 const uint64_t um = gs::ballot(upd);
                 taken = gs::write_lane(taken, (uint32_t)um | (uint32_t)(um >> 32), jj);
             }
@@ -2845,7 +2854,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
             blend_batch(std::integral_constant<bool, is_split(MODE)>{});
         else
             blend_batch(std::false_type{});
-        if constexpr (MODE != BLEND_GEO) {
+        if constexpr (has_marks(MODE)) {
             uint64_t m = km;
             if constexpr (is_split(MODE)) {
                 const uint64_t slots = gs::ballot(taken != 0u);
@@ -2861,7 +2870,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
         id_nxt = id_nn;
     }
 
-    if constexpr (MODE != BLEND_GEO) {
+    if constexpr (has_marks(MODE)) {
         const int nb = base < n ? base >> 6 : (n + 63) >> 6;   // batches walked
         put_masks(nb & ~63, nb);
     }
@@ -2880,7 +2889,7 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     if (inside) {
         const float Tf = __builtin_fabsf(px_st.T);
         O.final_T[pid] = Tf;
-        O.n_contrib_px[pid] = px_st.last;
+        O.n_contrib_px[pid] = MODE == BLEND_VIEW ? 0u : px_st.last;
         if (is_split(MODE)) O.n_contrib2loss_px[pid] = px_st.n2l;
         out_color[pid] = __builtin_fmaf(Tf, bg[0], px_st.C0);
         out_color[HW + pid] = __builtin_fmaf(Tf, bg[1], px_st.C1);
@@ -4352,6 +4361,10 @@ int render_forward_impl(int mode, int P, int64_t R, int W, int H, const float* b
         GS_TIMED("render_fwd_kernel", stream,
                  hipLaunchKernelGGL(render_fwd_kernel<BLEND_SPLIT>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
                                     NS, ranges, clist, recs, compute_locally, bg, O));
+    } else if (mode == BLEND_VIEW) {
+        GS_TIMED("render_fwd_kernel", stream,
+                 hipLaunchKernelGGL(render_fwd_kernel<BLEND_VIEW>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy, sgx,
+                                    NS, ranges, clist, recs, compute_locally, bg, O));
     } else if (mode == BLEND_SPLIT_GEO) {
         GS_TIMED("render_fwd_geo_kernel", stream,
                  hipLaunchKernelGGL(render_fwd_kernel<BLEND_SPLIT_GEO>, dim3(nblk), dim3(64), 0, stream, W, H, gx, gy,
@@ -4585,12 +4598,14 @@ extern "C" int gs_render_forward_count(int P, int W, int H, const float* means2D
                              stream, ~0ull, nullptr, region_side);
 }
 
-extern "C" int gs_render_forward(int P, int64_t R, int W, int H, const float* bg, const float* means2D,
-                                 const float* depths, const int* radii, const float* conic_opacity, const float* rgb,
-                                 const uint8_t* compute_locally, void* geom, void* binning, void* img,
-                                 float* out_color, int32_t* n_render, int32_t* n_consider, int32_t* n_contrib,
-                                 int32_t* out_observe, int region_side, void* clear_dst, int64_t clear_bytes,
-                                 hipStream_t stream)
+namespace {
+// the split forwards (BLEND_SPLIT, BLEND_VIEW)
+int split_forward(int mode, int P, int64_t R, int W, int H, const float* bg, const float* means2D,
+                  const float* depths, const int* radii, const float* conic_opacity, const float* rgb,
+                  const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                  float* out_color, int32_t* n_render, int32_t* n_consider, int32_t* n_contrib,
+                  int32_t* out_observe, int region_side, void* clear_dst, int64_t clear_bytes,
+                  hipStream_t stream)
 {
     gs::clear_error();
     GS_REQUIRE(n_render && n_consider && n_contrib && out_observe && out_color, "null output");
@@ -4600,19 +4615,19 @@ extern "C" int gs_render_forward(int P, int64_t R, int W, int H, const float* bg
     O.n_consider = n_consider;
     O.n_contrib_tile = n_contrib;
     if (int rc = clear_buf(clear_dst, clear_bytes, O.clr); rc != GS_OK) return rc;
-    return render_forward_impl(BLEND_SPLIT, P, R, W, H, bg, means2D, depths, radii, conic_opacity, rgb,
+    return render_forward_impl(mode, P, R, W, H, bg, means2D, depths, radii, conic_opacity, rgb,
                                compute_locally, nullptr, geom, binning, img, O, n_render, stream, nullptr,
                                region_side);
 }
 
-extern "C" int gs_render_forward_reserved(int P, int64_t capacity, int W, int H, const float* bg,
-                                          const float* means2D, const float* depths, const int* radii,
-                                          const float* conic_opacity, const float* rgb,
-                                          const uint8_t* compute_locally, void* geom, void* binning, void* img,
-                                          float* out_color, int32_t* n_render, int32_t* n_consider,
-                                          int32_t* n_contrib, int32_t* out_observe, int64_t* num_rendered,
-                                          int region_side, void* clear_dst, int64_t clear_bytes,
-                                          hipStream_t stream)
+int split_forward_reserved(int mode, int P, int64_t capacity, int W, int H, const float* bg,
+                           const float* means2D, const float* depths, const int* radii,
+                           const float* conic_opacity, const float* rgb,
+                           const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                           float* out_color, int32_t* n_render, int32_t* n_consider,
+                           int32_t* n_contrib, int32_t* out_observe, int64_t* num_rendered,
+                           int region_side, void* clear_dst, int64_t clear_bytes,
+                           hipStream_t stream)
 {
     gs::clear_error();
     GS_REQUIRE(n_render && n_consider && n_contrib && out_observe && out_color, "null output");
@@ -4624,10 +4639,63 @@ extern "C" int gs_render_forward_reserved(int P, int64_t capacity, int W, int H,
     if (int rc = clear_buf(clear_dst, clear_bytes, O.clr); rc != GS_OK) return rc;
     return reserved_forward(false, P, capacity, W, H, means2D, radii, compute_locally, nullptr, nullptr, geom,
                             num_rendered, stream, region_side, [&] {
-                                return render_forward_impl(BLEND_SPLIT, P, capacity, W, H, bg, means2D, depths, radii,
+                                return render_forward_impl(mode, P, capacity, W, H, bg, means2D, depths, radii,
                                                            conic_opacity, rgb, compute_locally, nullptr, geom, binning,
                                                            img, O, n_render, stream, nullptr, region_side);
                             });
+}
+}  // namespace
+
+extern "C" int gs_render_forward(int P, int64_t R, int W, int H, const float* bg, const float* means2D,
+                                 const float* depths, const int* radii, const float* conic_opacity, const float* rgb,
+                                 const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                                 float* out_color, int32_t* n_render, int32_t* n_consider, int32_t* n_contrib,
+                                 int32_t* out_observe, int region_side, void* clear_dst, int64_t clear_bytes,
+                                 hipStream_t stream)
+{
+    return split_forward(BLEND_SPLIT, P, R, W, H, bg, means2D, depths, radii, conic_opacity, rgb, compute_locally,
+                         geom, binning, img, out_color, n_render, n_consider, n_contrib, out_observe, region_side,
+                         clear_dst, clear_bytes, stream);
+}
+
+extern "C" int gs_render_forward_reserved(int P, int64_t capacity, int W, int H, const float* bg,
+                                          const float* means2D, const float* depths, const int* radii,
+                                          const float* conic_opacity, const float* rgb,
+                                          const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                                          float* out_color, int32_t* n_render, int32_t* n_consider,
+                                          int32_t* n_contrib, int32_t* out_observe, int64_t* num_rendered,
+                                          int region_side, void* clear_dst, int64_t clear_bytes,
+                                          hipStream_t stream)
+{
+    return split_forward_reserved(BLEND_SPLIT, P, capacity, W, H, bg, means2D, depths, radii, conic_opacity, rgb,
+                                  compute_locally, geom, binning, img, out_color, n_render, n_consider, n_contrib,
+                                  out_observe, num_rendered, region_side, clear_dst, clear_bytes, stream);
+}
+
+extern "C" int gs_render_view(int P, int64_t R, int W, int H, const float* bg, const float* means2D,
+                              const float* depths, const int* radii, const float* conic_opacity, const float* rgb,
+                              const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                              float* out_color, int32_t* n_render, int32_t* n_consider, int32_t* n_contrib,
+                              int32_t* out_observe, int region_side, void* clear_dst, int64_t clear_bytes,
+                              hipStream_t stream)
+{
+    return split_forward(BLEND_VIEW, P, R, W, H, bg, means2D, depths, radii, conic_opacity, rgb, compute_locally,
+                         geom, binning, img, out_color, n_render, n_consider, n_contrib, out_observe, region_side,
+                         clear_dst, clear_bytes, stream);
+}
+
+extern "C" int gs_render_view_reserved(int P, int64_t capacity, int W, int H, const float* bg,
+                                       const float* means2D, const float* depths, const int* radii,
+                                       const float* conic_opacity, const float* rgb,
+                                       const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                                       float* out_color, int32_t* n_render, int32_t* n_consider,
+                                       int32_t* n_contrib, int32_t* out_observe, int64_t* num_rendered,
+                                       int region_side, void* clear_dst, int64_t clear_bytes,
+                                       hipStream_t stream)
+{
+    return split_forward_reserved(BLEND_VIEW, P, capacity, W, H, bg, means2D, depths, radii, conic_opacity, rgb,
+                                  compute_locally, geom, binning, img, out_color, n_render, n_consider, n_contrib,
+                                  out_observe, num_rendered, region_side, clear_dst, clear_bytes, stream);
 }
 
 namespace {

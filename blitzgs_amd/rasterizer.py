@@ -311,8 +311,11 @@ class _PreprocessGaussians(torch.autograd.Function):
 
 def render_gaussians(means2D, means2D_abs, conic_opacity, rgb, all_map, depths, radii, compute_locally,
                      extended_compute_locally, raster_settings, cuda_args):
+    # without a gradient to take, the forward leaves nothing for a backward
+    backward = torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in
+                                               (means2D, means2D_abs, conic_opacity, rgb, all_map, depths))
     return _RenderGaussians.apply(means2D, means2D_abs, conic_opacity, rgb, all_map, depths, radii,
-                                  compute_locally, extended_compute_locally, raster_settings, cuda_args)
+                                  compute_locally, extended_compute_locally, raster_settings, cuda_args, backward)
 
 
 def _tile_mask(cl, H, W, device):
@@ -328,7 +331,7 @@ def _tile_mask(cl, H, W, device):
 
 
 def _render_forward_raw(bg, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, timing=False,
-                        debug=False, geo=None, region_side=None, clear=None):
+                        debug=False, geo=None, region_side=None, clear=None, backward=True):
     """Returns (num_rendered, color, n_render, n_consider, n_contrib, out_observe,
     geomBuffer, binningBuffer, imgBuffer, render_ms).  The binning buffer may be
     sized for more than num_rendered instances (_lib.InstanceReserve); render_ms
@@ -338,7 +341,9 @@ def _render_forward_raw(bg, H, W, means2D, depths, radii, conic_opacity, rgb, co
     region_side: the binning's region side (0, 2, 4, 8; None: chosen from the
     device's last forward, _lib.InstanceReserve.region_side).
     clear (without geo): a float32 device tensor, 16-byte aligned and a
-    multiple of 16 bytes, that the blend fills with zeros while it runs."""
+    multiple of 16 bytes, that the blend fills with zeros while it runs.
+    backward: False (without geo) leaves out of the buffers what only
+    _render_backward_raw reads."""
     _require_device(means2D, "means2D")
     dev = means2D.device
     P = means2D.size(0)
@@ -386,7 +391,8 @@ def _render_forward_raw(bg, H, W, means2D, depths, radii, conic_opacity, rgb, co
         args = (P, cap, W, H, ptr(bg), ptr(means2D), ptr(depths), ptr(radii), ptr(conic_opacity), ptr(rgb), ptr(cl),
                 ptr(geom), ptr(binning), ptr(img), *outs, C.byref(Rv))
         if maps is None:
-            check(lib.gs_render_forward_reserved(*args, rside, *clear_args, stream), "gs_render_forward_reserved")
+            forward = lib.gs_render_forward_reserved if backward else lib.gs_render_view_reserved
+            check(forward(*args, rside, *clear_args, stream), "gs_render_forward_reserved")
         else:
             check(lib.gs_render_forward_reserved_geo(*args, *geo_args, rside, stream),
                   "gs_render_forward_reserved_geo")
@@ -404,7 +410,8 @@ def _render_forward_raw(bg, H, W, means2D, depths, radii, conic_opacity, rgb, co
         args = (P, R, W, H, ptr(bg), ptr(means2D), ptr(depths), ptr(radii), ptr(conic_opacity), ptr(rgb), ptr(cl),
                 ptr(geom), ptr(binning), ptr(img), *outs)
         if maps is None:
-            check(lib.gs_render_forward(*args, rside, *clear_args, stream), "gs_render_forward")
+            forward = lib.gs_render_forward if backward else lib.gs_render_view
+            check(forward(*args, rside, *clear_args, stream), "gs_render_forward")
         else:
             check(lib.gs_render_forward_geo(*args, *geo_args, rside, stream), "gs_render_forward_geo")
     _lib.debug_sync(debug, "gs_render_forward")
@@ -501,7 +508,7 @@ def _render_backward_raw(bg, R, H, W, means2D, conic_opacity, rgb, compute_local
 class _RenderGaussians(torch.autograd.Function):
     @staticmethod
     def forward(ctx, means2D, means2D_abs, conic_opacity, rgb, all_maps, depths, radii, compute_locally,
-                extended_compute_locally, raster_settings, cuda_args):
+                extended_compute_locally, raster_settings, cuda_args, backward=True):
         rs = raster_settings
         render_geo = bool(getattr(rs, "render_geo", False))
         if render_geo and (all_maps is None or tuple(all_maps.shape) != (means2D.size(0), 5)):
@@ -524,7 +531,7 @@ class _RenderGaussians(torch.autograd.Function):
             n = 6 * H * W
             zmaps = torch.empty(((n + 3) // 4) * 4, device=means2D.device, dtype=torch.float32)
         res = _render_forward_raw(rs.bg, H, W, means2D, depths, radii, conic_opacity, rgb, cl, timing,
-                                  bool(rs.debug), geo=geo, clear=zmaps)
+                                  bool(rs.debug), geo=geo, clear=zmaps, backward=backward)
         # the preprocess backward's dL/dsh, which this render's backward clears
         zg = getattr(means2D, "_gs_zeroed", None)
         ctx.zeroed = zg if isinstance(zg, _ZeroedGrads) else None
@@ -580,7 +587,7 @@ class _RenderGaussians(torch.autograd.Function):
         if not ctx.needs_input_grad[4]:
             dL_dall_map = None
         return (dL_dmeans2D, dL_dmeans2D_abs, dL_dconic_opacity, dL_dcolors, dL_dall_map,
-                None, None, None, None, None, None)
+                None, None, None, None, None, None, None)
 
 
 class GaussianRasterizer(nn.Module):

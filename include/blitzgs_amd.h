@@ -219,6 +219,26 @@ int gs_render_forward_reserved(int P, int64_t capacity, int image_width, int ima
                                int region_side, void* clear_dst, int64_t clear_bytes,
                                gs_stream_t stream);
 
+/* gs_render_forward / gs_render_forward_reserved for a view that no backward
+ * follows: the same arguments, outputs and lists, without what only
+ * gs_render_backward reads (the marks of the blended entries in `binning`; the
+ * contributor counts in `img` are zero, and a backward over them returns zeros).
+ * Repeat a gs_render_view_reserved that did not fit with gs_render_view. */
+int gs_render_view(int P, int64_t R, int image_width, int image_height, const float* bg,
+                   const float* means2D, const float* depths, const int* radii,
+                   const float* conic_opacity, const float* rgb, const uint8_t* compute_locally,
+                   void* geom, void* binning, void* img, float* out_color, int32_t* n_render,
+                   int32_t* n_consider, int32_t* n_contrib, int32_t* out_observe,
+                   int region_side, void* clear_dst, int64_t clear_bytes, gs_stream_t stream);
+int gs_render_view_reserved(int P, int64_t capacity, int image_width, int image_height,
+                            const float* bg, const float* means2D, const float* depths,
+                            const int* radii, const float* conic_opacity, const float* rgb,
+                            const uint8_t* compute_locally, void* geom, void* binning, void* img,
+                            float* out_color, int32_t* n_render, int32_t* n_consider,
+                            int32_t* n_contrib, int32_t* out_observe, int64_t* num_rendered,
+                            int region_side, void* clear_dst, int64_t clear_bytes,
+                            gs_stream_t stream);
+
 /* Render backward.  Replaces RenderGaussiansBackwardCUDA
  * (diff-gaussian-rasterization_r/rasterize_points.cu:363-436; kernel
  * cuda_rasterizer/backward.cu:324-530).
