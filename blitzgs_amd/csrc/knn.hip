@@ -205,26 +205,36 @@ __device__ __forceinline__ void upd3(float& b0, float& b1, float& b2, float d)
     b2 = n2;
 }
 
-// candidates sorted[lo, hi) against the query at sorted position `self`; four
-// loads in flight, the last four clamped to the segment and masked
+// candidates sorted[k, k + 4) against the query, four loads in flight.  TAIL:
+// those from hi on are masked (and their loads clamped); OWN: so is the query
+// itself, at sorted position `self`, which only its own run of cells holds.
+// The masks are half of a candidate's VALU instructions, which bind where the
+// runs are long (points with a few far outliers, whose bulk shares a few cells):
+// 100k points, three of them far away, 45.8 ms with both masks on every
+// candidate, 35.4 ms so; without outliers 0-8 % faster.
+template <bool TAIL, bool OWN>
 __device__ __forceinline__ void scan_four(uint32_t k, uint32_t hi, const float4* __restrict__ sorted, float4 q,
                                           uint32_t self, float& b0, float& b1, float& b2)
 {
     float4 o[4];
 #pragma unroll
-    for (uint32_t u = 0; u < 4; u++) o[u] = sorted[min(k + u, hi - 1)];
+    for (uint32_t u = 0; u < 4; u++) o[u] = sorted[TAIL ? min(k + u, hi - 1) : k + u];
 #pragma unroll
     for (uint32_t u = 0; u < 4; u++) {
         const float dx = o[u].x - q.x, dy = o[u].y - q.y, dz = o[u].z - q.z;
         const float d = (dx * dx + dy * dy) + dz * dz;
-        upd3(b0, b1, b2, k + u >= hi || k + u == self ? __builtin_huge_valf() : d);
+        upd3(b0, b1, b2, (TAIL && k + u >= hi) || (OWN && k + u == self) ? __builtin_huge_valf() : d);
     }
 }
 
+// candidates sorted[lo, hi)
+template <bool OWN>
 __device__ __forceinline__ void scan_segment(uint32_t lo, uint32_t hi, const float4* __restrict__ sorted, float4 q,
                                              uint32_t self, float& b0, float& b1, float& b2)
 {
-    for (uint32_t k = lo; k < hi; k += 4) scan_four(k, hi, sorted, q, self, b0, b1, b2);
+    uint32_t k = lo;
+    for (; k + 4 <= hi; k += 4) scan_four<false, OWN>(k, hi, sorted, q, self, b0, b1, b2);
+    if (k < hi) scan_four<true, OWN>(k, hi, sorted, q, self, b0, b1, b2);
 }
 
 // What a point `gap` cells beyond the neighbouring cell keeps from the query
@@ -273,9 +283,10 @@ __device__ __forceinline__ bool box_done(double bound, float b2)
 // total, not the sum over the runs of the longest lane in each.  Only if the
 // third-best distance is not yet provably final are further shells visited,
 // again without the rows that lie beyond it.  Bound by the latency of the
-// gathered candidates and by the longest lane of a wave.  10M points of a ground
-// plane with dense clusters: 4.96 ms with every run scanned in turn (3 points per
-// cell), 3.45 ms so at the same cells.
+// gathered candidates and by the longest lane of a wave; by VALU issue where a
+// cell holds hundreds of points.  10M points of a ground plane with dense
+// clusters, whole call at 3 points per cell: 6.1 ms with every run scanned in
+// turn, 4.3 ms so.
 __global__ __launch_bounds__(QT) void knn_query_kernel(int P, Grid g, const uint32_t* __restrict__ start,
                                                        const float4* __restrict__ sorted, float* __restrict__ out)
 {
@@ -301,7 +312,7 @@ __global__ __launch_bounds__(QT) void knn_query_kernel(int P, Grid g, const uint
     {
         const int x0 = max(0, c[0] - 1), x1 = min(g.n[0] - 1, c[0] + 1);
         const uint32_t own = (uint32_t)((c[2] * g.n[1] + c[1]) * g.n[0]);
-        scan_segment(start[own + (uint32_t)x0], start[own + (uint32_t)x1 + 1], sorted, q, self, b0, b1, b2);
+        scan_segment<true>(start[own + (uint32_t)x0], start[own + (uint32_t)x1 + 1], sorted, q, self, b0, b1, b2);
         float lo2[3], hi2[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -343,7 +354,10 @@ __global__ __launch_bounds__(QT) void knn_query_kernel(int P, Grid g, const uint
                 i++;
             }
             if (k >= e) break;
-            scan_four(k, e, sorted, q, self, b0, b1, b2);
+            if (gs::ballot(k + 4 > e) == 0)   // no lane at its segment's end
+                scan_four<false, false>(k, e, sorted, q, self, b0, b1, b2);
+            else
+                scan_four<true, false>(k, e, sorted, q, self, b0, b1, b2);
             k += 4;
         }
     }
@@ -367,17 +381,17 @@ __global__ __launch_bounds__(QT) void knn_query_kernel(int P, Grid g, const uint
                     const bool shell_zy = (z == c[2] - r || z == c[2] + r || y == c[1] - r || y == c[1] + r);
                     if (shell_zy) {
                         // the whole x run of this shell row is new: one segment
-                        scan_segment(start[row + (uint32_t)xa], start[row + (uint32_t)xb + 1], sorted, q, self, b0,
-                                     b1, b2);
+                        scan_segment<false>(start[row + (uint32_t)xa], start[row + (uint32_t)xb + 1], sorted, q, self,
+                                            b0, b1, b2);
                     } else {
                         // interior rows: only the two x ends are new
                         if (c[0] - r >= 0 && !(b2 < gy + xlo2)) {
                             const uint32_t cc = row + (uint32_t)(c[0] - r);
-                            scan_segment(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
+                            scan_segment<false>(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
                         }
                         if (c[0] + r < g.n[0] && !(b2 < gy + xhi2)) {
                             const uint32_t cc = row + (uint32_t)(c[0] + r);
-                            scan_segment(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
+                            scan_segment<false>(start[cc], start[cc + 1], sorted, q, self, b0, b1, b2);
                         }
                     }
                 }
@@ -433,9 +447,11 @@ int knn_impl(int P, const float* points, float* out, void* workspace, hipStream_
     }
     // about 4.5 points per cell: coarser cells spare the points in the sparse parts
     // their shells, and the query skips what they add elsewhere (measured, whole
-    // call, at 2 / 3 / 4.5 / 6 / 8 per cell: 10M points of a ground plane with dense
-    // clusters 4.82 / 3.97 / 3.61 / 3.62 / 3.78 ms, 100k in clusters
-    // 157 / 133 / 136 / 162 / 165 us, 1M uniform 204 / 208 / 205 / 209 / 205 us),
+    // call, at 2 / 3 / 4.5 per cell: 10M points of a ground plane with dense clusters
+    // 5.15 / 4.30 / 3.82 ms, 5M in clusters 2.13 / 1.70 / 1.50 ms, 1M uniform
+    // 205 / 198 / 197 us, 2M on a sphere 0.54 / 0.61 / 0.70 ms; at 6 and 8 the 10M
+    // take 0 and 5 % longer).  Points with a few far outliers take 24 to 33 ms per 100k
+    // at any of them, by where the cell faces fall in their bulk,
     // at most 1024 cells per axis and max_cells(P) in total
     double h = cbrt(vol / ((double)P / 4.5 + 1.0));
     size_t NC = 0;

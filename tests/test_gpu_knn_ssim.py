@@ -37,7 +37,7 @@ def test_knn_bitexact(n, kind):
     assert_bitexact(got, ref, f"distCUDA2 {kind} n={n}")
 
 
-@pytest.mark.parametrize("kind", ["lattice", "one_cluster", "offset", "line", "pairs"])
+@pytest.mark.parametrize("kind", ["lattice", "one_cluster", "outliers", "offset", "line", "pairs"])
 @pytest.mark.parametrize("n", [63, 4097, 30011])
 def test_knn_skipped_rows_bitexact(n, kind):
     # points whose neighbours lie in skipped or trimmed rows if a bound is too
@@ -50,6 +50,9 @@ def test_knn_skipped_rows_bitexact(n, kind):
         pts = np.stack(np.meshgrid(*[np.arange(k)] * 3), -1).reshape(-1, 3)[:n] * 0.25
     elif kind == "one_cluster":
         pts = np.concatenate([rng.normal(0, 0.01, (n - n // 50, 3)), rng.uniform(-10, 10, (n // 50, 3))])
+    elif kind == "outliers":   # nearly all points in a few cells: long runs, every remainder of four
+        pts = rng.normal(0, 1, (n, 3))
+        pts[:3] *= 300
     elif kind == "offset":
         pts = rng.uniform(0, 1, (n, 3)) + np.array([1000.0, -3000.0, 7.0])
     elif kind == "line":
