@@ -167,17 +167,6 @@ extern "C" int gs_version(void) { return 100; }
 extern "C" const char* gs_last_error(void) { return g_err; }
 
 namespace {
-// op 3: x holds 12 x 64 values ([value][lane]); y[k] = sum over lanes of value k
-__global__ void diag_sum12_kernel(const float* __restrict__ x, float* __restrict__ y)
-{
-    float v[12];
-#pragma unroll
-    for (int k = 0; k < 12; k++) v[k] = x[k * 64 + threadIdx.x];
-    const float t = gs::wave_sum12(v);
-    const int k = gs::wave_sum12_index((int)threadIdx.x);
-    if (k >= 0) y[k] = t;
-}
-
 __global__ void diag_math_kernel(int op, int n, const float* __restrict__ x, float* __restrict__ y)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -226,9 +215,9 @@ extern "C" int gs_diag_math(int op, int n, const float* x, float* y, hipStream_t
 {
     gs::clear_error();
     GS_REQUIRE(op >= 0 && op <= 9,
-               "op must be 0 (exp), 1 (log), 2 (exact blend exp), 3 (wave sum of 12 values), 4 (copy), "
-               "5 (VALU rate), 6 (the blend's falloff G), 7, 8 or 9 (forward / backward / half-tile backward "
-               "blend VALU probe)");
+               "op must be 0 (exp), 1 (log), 2 (exact blend exp), 3 (wave sums of 12 values), 4 (copy), "
+               "5 (VALU rate), 6 (the blend's falloff G), 7, 8 or 9 (forward / backward / backward blend "
+               "VALU probe)");
     GS_REQUIRE(n >= 0, "n must be >= 0");
     if (op >= 7 && op <= 9) return gs::render_valu_probe(op - 7, n, y, stream);
     if (op == 5) {
@@ -242,9 +231,7 @@ extern "C" int gs_diag_math(int op, int n, const float* x, float* y, hipStream_t
     }
     if (op == 3) {
         GS_REQUIRE(n == 12 * 64, "op 3 takes 12 x 64 inputs");
-        hipLaunchKernelGGL(diag_sum12_kernel, dim3(1), dim3(64), 0, stream, x, y);
-        GS_LAUNCH_CHECK("diag_sum12_kernel");
-        return GS_OK;
+        return gs::render_grad_reduce(x, y, stream);
     }
     if (n == 0) return GS_OK;
     if (op == 4) {

@@ -22,8 +22,10 @@ void timing_mark_end(hipStream_t stream);
 // its time runs from the begin mark to the end mark of the same name.
 void timing_stage_begin(hipStream_t stream, const char* name);
 void timing_stage_end(hipStream_t stream, const char* name);
-// The blend kernels' VALU probes (render.hip): which 0 forward, 1 backward.
+// The blend kernels' VALU probes (render.hip): which 0 forward, 1 or 2 backward.
 int render_valu_probe(int which, int iters, float* y, hipStream_t stream);
+// The render backward's reduction of 12 x 64 values (render.hip).
+int render_grad_reduce(const float* x, float* y, hipStream_t stream);
 }  // namespace gs
 
 #define GS_TIMED(name, stream, launch)                                                 \

@@ -2665,7 +2665,8 @@ struct ClearAtExit {
 // entries marked), forward 263 -> 283 us (267 us); at 1M wide ones, 1920x1080:
 // 286 -> 260 us and 174 -> 187 us.  The evaluation views of the full-image
 // path run no backward, so that path takes the cheaper mark (forward 221 ->
-// 222 us at 6M; with the other 241 us).
+// 222 us at 6M; with the other 241 us); the split path's views take none
+// (BLEND_VIEW).
 struct StagedMasks {
     uint64_t* full;   // 4 words (quadrants) per 64 positions, in the binning buffer
     uint64_t* tail;   // 4 words per tile
@@ -2700,8 +2701,9 @@ struct FwdOut {
 };
 
 template <int MODE>
-// (waves per SIMD: eight fit in 64 VGPRs without spills in the loop;
-// render_geo's maps and their LDS leave six or seven)
+// (waves per SIMD: eight fit in 64 VGPRs; the full-image modes spill one pair
+// around the loop, none inside it.  render_geo's colour walk takes 72 VGPRs for
+// its five more sums: seven waves)
 __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
@@ -2748,8 +2750,12 @@ __global__ __launch_bounds__(64, is_geo(MODE) ? 6 : 8) void render_fwd_kernel(
 
     // the list entries of the next two batches are in flight while one blends.
     // Their records are not: the registers they would hold cost two waves per
-    // SIMD, which hide their latency better.  Measured: 6M aerial Gaussians at
-    // 1600x1066 272 -> 263 us (the full-image path's blend 232 -> 221 us)
+    // SIMD, which hide their latency better once there are that many.  Measured,
+    // records in flight -> not: 6M aerial Gaussians at 1600x1066 272 -> 263 us (the
+    // full-image path's blend 232 -> 221 us), 1M wide ones at 1920x1080 201 ->
+    // 193 us, 300k at 800x600 101 -> 99 us; with fewer than about five waves per
+    // SIMD the other way round, 60k at 512x512 65 -> 68 us, 16k at 256x256 64 ->
+    // 66 us, which is not worth a second variant of the kernel
     uint32_t id_cur = lane < n ? list[lane] : 0u;
     uint32_t id_nxt = 64 + lane < n ? list[64 + lane] : 0u;
     // the staged masks of up to 64 batches, batch b in lane b % 64 (written
@@ -3381,17 +3387,19 @@ __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, co
 // Bound: the walk is bound by VALU issue.  Forming the eleven terms per pixel
 // and summing each over 64 lanes by transpose-adds made an entry 82 VALU
 // instructions; this makes it 60 (58 with the moments; counted on the probe).
-// Measured (render
-// backward, before -> after): 6M aerial Gaussians at 1600x1066 642 -> 510 us,
-// 1M wide ones at 1920x1080 367 -> 284 us, the full-image path's 2M at
-// 1237x822 377 -> 225 us.  Tried: the sums as a contraction on the matrix
+// Measured
+// (render backward, per pixel -> with the moments; in brackets now, with the
+// offsets one by one and the marks): 6M aerial Gaussians at 1600x1066 642 ->
+// 510 us (437), 1M wide ones at 1920x1080 367 -> 284 us (267), the full-image
+// path's 2M at 1237x822 377 -> 225 us (235); render_geo's 6M 909 us (600), 1M
+// 565 us (350).  Tried: the sums as a contraction on the matrix
 // cores, v_mfma_f32_16x16x4_f32 with four entries' rows against per-pixel
 // constants (equal accuracy): 700 us at 6M, because a float32 MFMA and the
 // VALU do not overlap on this target (a loop of one MFMA and 16 FMAs takes 108
 // cycles, of either alone 34 and 71; a bf16 MFMA does overlap, but splitting
 // the rows into three bf16 parts costs more VALU than it saves); eight entries
 // of eight pixels per lane (fewer instructions, but four waves per SIMD and
-// twice the accumulator lines per entry): 422 -> 508 us at 6M.
+// twice the accumulator lines per entry): 508 -> 594 us at 6M, before the marks.
 constexpr int GRAD_SLOTS = 4;          // entries per flush
 constexpr int GRAD_STRIDE = 3 * 64 + 8;   // floats per slot: 3 rows, and 8 more so that 8 lanes' 16-byte reads meet 32 banks
 
@@ -4902,8 +4910,35 @@ extern "C" int gs_render_full_backward(int P, int64_t R, int W, int H, const flo
                                 dL_dmeans2D, 3, nullptr, dL_dconic_opacity, dL_dcolors, stream);
 }
 
+namespace {
+// x holds 12 x 64 values ([value][lane]); y[k] = the sum over the lanes of
+// value k: grad_reduce's slots, its four entries' sums added
+__global__ __launch_bounds__(64) void grad_reduce_kernel(const float* __restrict__ x, float* __restrict__ y)
+{
+    const int lane = threadIdx.x;
+    float p[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const float a = k < 6 ? x[2 * k * 64 + lane] : 0.f, b = k < 6 ? x[(2 * k + 1) * 64 + lane] : 0.f;
+        p[k] = swap32_add(a, b);
+    }
+    float v = grad_reduce<true>(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], lane);
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 4, 64);
+    const int i = grad_slot(lane);
+    if (((lane >> 1) & 3) == 0 && i < 12) y[i] = v;
+}
+}  // namespace
+
 namespace gs {
-// The VALU probes (which 0: forward, 1: backward) over `iters` passes of 64
+int render_grad_reduce(const float* x, float* y, hipStream_t stream)
+{
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3(1), dim3(64), 0, stream, x, y);
+    GS_LAUNCH_CHECK("grad_reduce_kernel");
+    return GS_OK;
+}
+
+// The VALU probes (which 0: forward, 1 or 2: backward) over `iters` passes of 64
 // entries per wave, VALU_PROBE_BLOCKS waves.
 int render_valu_probe(int which, int iters, float* y, hipStream_t stream)
 {

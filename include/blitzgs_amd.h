@@ -625,14 +625,15 @@ int gs_ply_pack(int64_t P, int32_t n_tensors, const gs_ply_tensor* tensors, cons
  * Diagnostics (no counterpart in the reference): evaluate the device exp / log
  * used by the kernels on n inputs (op 0 = exp, 1 = log, 2 = the exact exp of
  * the blend's guard,
- * 3 = the 12-value wave reduction on 12 x 64 inputs), so tests can compare them
+ * 3 = the sums over the wave of 12 values per lane, 12 x 64 inputs, by the
+ * render backward's reduction), so tests can compare them
  * bit for bit with the CPU; op 6 evaluates the blend's falloff G = exp(x),
  * x <= 0 (hardware exp2, exact within a window around the 1/255 alpha
  * cut-off at opacity 1); op 4 copies n floats (n % 4 == 0, 16-byte aligned),
  * the known-size kernel that HBM byte counters are calibrated against; op 5
  * runs 8192 blocks of 256 threads, each wave issuing 32 * n fp32 FMAs (x unused,
  * y one float that is never written), the reference for the VALU issue rate;
- * ops 7 and 8 (and 9, the same as 8) run the forward / backward blend
+ * ops 7 and 8 (9 is the same as 8) run the forward / backward blend
  * kernels' per-entry arithmetic (the same device functions) n times over 64
  * entries staged in LDS, in 16384 waves with no global memory traffic (x
  * unused, y one float that is never written): the VALU issue rate of the

@@ -48,8 +48,8 @@ def _cuda_args(avoid):
 
 
 def _scene(wide=False):
-    # wide: Gaussians with ~67 tile instances each, for which the backward
-    # walks 16x8 half tiles, two pixels per lane
+    # wide: Gaussians with ~67 tile instances each, i.e. long lists of which a
+    # quadrant blends most
     if wide:
         scene, cam = synth.small_scene(2500, seed=64, W=287, H=213, extent=1.4, log_mu=-1.2)
     else:

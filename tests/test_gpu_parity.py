@@ -49,9 +49,9 @@ def test_device_math_bitexact():
 
 
 def test_valu_probes_run_and_write_nothing():
-    """The blend kernels' VALU probes (gs_diag_math ops 7, 8 and 9: forward,
-    quadrant backward, half-tile backward) run, and the float they could
-    write stays untouched (the work is kept alive by a test that never
+    """The blend kernels' VALU probes (gs_diag_math ops 7 and 8: forward,
+    backward; 9 is the same as 8) run, and the float they could write stays
+    untouched (the work is kept alive by a test that never
     holds)."""
     y = torch.zeros(1, device="cuda")
     for op in (7, 8, 9):
@@ -592,9 +592,9 @@ def test_autograd_clears_preprocess_grads_beside_the_render(monkeypatch):
 @pytest.mark.parametrize("cfg", ["small", "config0", "wide"])
 def test_autograd_forward_backward_vs_oracle(cfg):
     """The autograd pair against the oracle's chain.  "wide": Gaussians with
-    more than 24 tile instances each on average, for which the backward walks
-    16x8 half tiles with two pixels per lane instead of 8x8 quadrants (the
-    200x150 image leaves partial tiles on both edges)."""
+    more than 24 tile instances each on average: long lists of which a
+    quadrant blends most (the 200x150 image leaves partial tiles on both
+    edges)."""
     from blitzgs_amd import rasterizer as R
     if cfg == "small":
         scene, cam = synth.small_scene(3000, seed=12, W=200, H=150, extent=1.2)
@@ -708,9 +708,9 @@ def test_quadrant_cull_keeps_results_exact_on_hard_cases():
 
 
 def test_wave_sum12_lane_layout():
-    # the backward's 12-value wave reduction (permlane32/16 swaps, then DPP
-    # transpose-adds) against a plain sum, with values that make any mis-routed
-    # lane visible
+    # the render backward's reduction (permlane32/16 swaps, then DPP
+    # transpose-adds; its four entries' sums added) against a plain sum, with
+    # values that make any mis-routed lane visible
     rng = np.random.default_rng(0)
     x = rng.integers(-1000, 1000, (12, 64)).astype(np.float32)
     x[7] = 1.0
