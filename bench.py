@@ -30,8 +30,10 @@ launch stream inside the timed region; `cpu_baseline` times the CPU oracle
 host.
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -302,16 +304,34 @@ def valu_probes_only():
         log(f"[bench] {pname}: {iters} iterations, {ms:.3f} ms")
 
 
+def kernel_code():
+    """Hash of the step's kernel sources without their comments.  A counter file
+    of profiles/ holds the one it was taken at ("code"): counts of other kernels
+    are not divided by the times of these."""
+    h = hashlib.sha256()
+    for f in ("render.hip", "preprocess.hip", "gs_device.h"):
+        text = re.sub(r"//[^\n]*", "", open(os.path.join(ROOT, "blitzgs_amd", "csrc", f)).read())
+        h.update("".join(text.split()).encode())
+    return h.hexdigest()[:16]
+
+
+def step_counts(name):
+    """profiles/<name>.json, or {} when it is absent or of other kernels."""
+    try:
+        counts = json.load(open(os.path.join(ROOT, "profiles", name + ".json")))
+    except (OSError, ValueError):
+        return {}
+    return counts if counts.get("code") == kernel_code() else {}
+
+
 def valu_of(name, avg_ms, config):
     """VALU issue rate of kernel `name` per launch: SQ_INSTS_VALU per launch
     (profiles/valu_config<N>.json, rocprofv3 --pmc) over its live launch time,
     against the ceiling for its instruction mix: the issue rate of its VALU
     probe (the same per-entry arithmetic with no memory traffic; instructions
     per probe launch in profiles/valu_probes.json, the probe timed live)."""
-    f = os.path.join(ROOT, "profiles", f"valu_config{config}.json")
-    try:
-        insts = json.load(open(f))[name]["SQ_INSTS_VALU"]
-    except (OSError, ValueError, KeyError):
+    insts = step_counts(f"valu_config{config}").get(name, {}).get("SQ_INSTS_VALU")
+    if insts is None:
         return None
     achieved = insts / (avg_ms * 1e-3) / 1e9
     out = {"unit": "G wave-instructions/s", "insts_per_launch": int(insts), "achieved": round(achieved, 1),
@@ -319,13 +339,13 @@ def valu_of(name, avg_ms, config):
     if name in VALU_PROBES:
         op, pname, iters = VALU_PROBES[name]
         try:
-            pj = json.load(open(os.path.join(ROOT, "profiles", "valu_probes.json")))[pname]
+            pj = step_counts("valu_probes")[pname]
             assert int(pj["iters"]) == iters
             peak = pj["SQ_INSTS_VALU"] / (run_valu_probe(op, iters) * 1e-3) / 1e9
             out.update(peak=round(peak, 1), frac=round(achieved / peak, 4),
                        peak_is=f"measured VALU issue rate of the kernel's own per-entry arithmetic "
                                f"({pname}, gs_diag_math op {op}: no memory traffic, {iters} x 64 entries per wave)")
-        except (OSError, ValueError, KeyError, AssertionError):
+        except (KeyError, AssertionError):
             pass
     return out
 
@@ -435,13 +455,7 @@ def run_step(args):
         for k, v in sorted(per_kernel.items(), key=lambda x: -x[1]):
             log(f"[bench]   {k:28s} {v:8.4f} ms/step  ({kt[k][1] // max(1, args.steps)} launches)")
     dom = max(STEP_STAGES + ("binning",), key=lambda k: stages.get(k, 0.0))
-    traffic = None
-    tf = os.path.join(ROOT, "profiles", f"traffic_config{args.config}.json")
-    if os.path.exists(tf):
-        try:
-            traffic = json.load(open(tf)).get(dom)
-        except (OSError, ValueError):
-            traffic = None
+    traffic = step_counts(f"traffic_config{args.config}").get(dom)
     roofline = roofline_of(dom, sb[dom], avg_launch.get(dom, float("nan")), traffic)
     if dom == "binning":
         roofline["note"] = ("binning = tile count, scan, duplication and the per-tile sorts, timed as one stage on "

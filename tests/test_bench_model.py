@@ -56,3 +56,14 @@ def test_region_entries_match_enumeration(bench, rows, side):
     got = bench.region_entries(torch.from_numpy(m), torch.from_numpy(r), W, H, cl, side=side)
     assert got == _enumerate(m, r, W, H, rows, max(side, 2))
     assert got > 1000
+
+
+def test_counts_of_other_kernels_are_not_used(bench, monkeypatch):
+    """The instruction and traffic counts of profiles/ are those of the kernels
+    in the tree, and are left out for any other."""
+    for f in ("valu_config1", "valu_config2", "valu_probes", "traffic_config1", "traffic_config2"):
+        assert bench.step_counts(f), f
+    assert bench.step_counts("no_such_file") == {}
+    monkeypatch.setattr(bench, "kernel_code", lambda: "other")
+    assert bench.step_counts("valu_config2") == {}
+    assert bench.valu_of("render_bwd_kernel", 0.5, 2) is None
