@@ -151,8 +151,8 @@ int gs_preprocess_backward_rec_acc(int P, int D, int K, const void* bwd_records,
  *
  *   geom    : gs_render_geom_bytes(P, W, H) bytes  (counts, offsets)
  *   binning : gs_render_binning_bytes(R) bytes     (the blend's sorted list;
- *             the point list and its keys on request; a buffer sized for a
- *             capacity >= R serves R)
+ *             the point list and its keys on request; the marks of the entries
+ *             the backward walks; a buffer sized for a capacity >= R serves R)
  *   img     : gs_render_img_bytes(W, H) bytes      (tile ranges, per-pixel
  *             final transmittance and contributor counts)
  * compute_locally is a uint8 (ceil(H/16), ceil(W/16)) tile mask, or NULL
@@ -244,7 +244,8 @@ int gs_render_view_reserved(int P, int64_t capacity, int image_width, int image_
  * cuda_rasterizer/backward.cu:324-530).
  *   geom / binning / img: the forward's workspaces (geom also holds the
  *   gradient accumulators, cleared at the start of each call, so calls
- *   sharing one geom must not overlap).  means2D / conic_opacity / rgb: the forward's inputs
+ *   sharing one geom must not overlap; of binning the call reads the list and
+ *   the forward's marks at its end, so it needs the whole buffer).  means2D / conic_opacity / rgb: the forward's inputs
  *   (the kernels read the forward's packed copy of them in geom).
  *   dL_dpixels (3,H,W).  Outputs: dL_dmeans2D (row stride dL_dmeans2D_stride,
  *   2 or 3; the third column, when present, is zero), dL_dmeans2D_abs (P,3),
