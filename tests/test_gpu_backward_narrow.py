@@ -83,7 +83,6 @@ def _reference(x, full, geo):
     T = after / (1 - al)
     e = 3e-6 + 3e-7 * use.sum(0) + 6e-7 * (al / (1 - al)).sum(0)
     free = use & (oG <= CLAMP) if full else use
-    assert not full or (use & ~free).sum() >= 8
     out = []
     for ab in (lambda v: v, np.abs):
         cd = ab(col) @ ab(dL)
@@ -132,7 +131,7 @@ def _full(x, dL=None):
     s = _lib.stream_of(dev)
     m, c, g, bg, d, rad = (to_dev(x[k]) for k in ("means2D", "conic", "rgb", "bg", "depths", "radii"))
     P = m.shape[0]
-    rects = torch.full((P, 2), float(x["radii"][0]), device=dev)
+    rects = rad.float()[:, None].expand(P, 2).contiguous()
     buf = lambda n: torch.empty(int(n), device=dev, dtype=torch.uint8)  # noqa: E731
     f32 = lambda *shape: torch.empty(shape, device=dev)  # noqa: E731
     geom, img, color = buf(lib.gs_render_geom_bytes(P, W, H)), buf(lib.gs_render_img_bytes(W, H)), f32(3, H, W)
@@ -148,11 +147,8 @@ def _full(x, dL=None):
     return dict(m2=dm[:, :2], con=dc, col=dg)
 
 
-@pytest.mark.parametrize("path", ["split", "geo", "full"])
-@pytest.mark.parametrize("seed,faint", [(0, False), (1, True), (2, True)])
-def test_narrow(gpu, path, seed, faint):
+def _check(x, path):
     full, geo = path == "full", path == "geo"
-    x = _inputs(seed, clamped=full, faint=faint)
     ref, bound = _reference(x, full, geo)
     got = _full(x) if full else _split(x, geo)
     assert set(got) == set(ref)
@@ -162,6 +158,34 @@ def test_narrow(gpu, path, seed, faint):
         bad = np.abs(g - ref[k]) > bound[k]
         i = np.unravel_index((np.abs(g - ref[k]) / np.maximum(bound[k], 1e-300)).argmax(), g.shape)
         assert int(bad.sum()) == 0, (k, int(bad.sum()), i, g[i], ref[k][i], bound[k][i])
+
+
+@pytest.mark.parametrize("path", ["split", "geo", "full"])
+@pytest.mark.parametrize("seed,faint", [(0, False), (1, True), (2, True)])
+def test_narrow(gpu, path, seed, faint):
+    _check(_inputs(seed, clamped=path == "full", faint=faint), path)
+
+
+@pytest.mark.parametrize("path", ["split", "geo", "full"])
+def test_blended_entries_far_apart_in_a_long_list(gpu, path):
+    """130 Gaussians that every pixel blends among 9000 that lie between pixel
+    centres of one quadrant of two tiles and are blended by none: lists of more
+    than 64 batches of 64, most of whose marks are empty (split) or staged in vain
+    (full)."""
+    n, wide = 9130, 130
+    rng = np.random.default_rng(5)
+    x = _inputs(5, n=n)
+    m = np.where(np.arange(n)[:, None] % 2 == 0, [3.5, 3.5], [35.5, 19.5]) + rng.uniform(-0.1, 0.1, (n, 2))
+    s = 1 / 0.3
+    conic = np.stack([np.full(n, s), np.zeros(n), np.full(n, s), rng.uniform(1.05, 1.3, n) / 255], 1)
+    radii = np.full(n, 2, np.int32)
+    at = rng.choice(n, wide, replace=False)
+    m[at] = rng.uniform([0, 0], [W, H], (wide, 2))
+    conic[at] = np.stack([np.full(wide, 1 / 60 ** 2), np.zeros(wide), np.full(wide, 1 / 45 ** 2),
+                          rng.uniform(0.012, 0.03, wide)], 1)
+    radii[at] = 2000
+    x.update(means2D=m.astype(np.float32), conic=conic.astype(np.float32), radii=radii)
+    _check(x, path)
 
 
 @pytest.mark.parametrize("value", [np.nan, np.inf])

@@ -4,8 +4,9 @@ out in float64.
 
 n Gaussians that every pixel of a 40x24 image blends (partial tiles on two
 edges), so that each quadrant's walk has n entries: remainders of four, of the
-64 staged at a time and of the 64-position list words; narrow and very wide
-ones, some with their means far outside the image.
+64 staged at a time and of the 64-position list words; ones as wide as the
+image and ten times wider, some with their means far outside it.  (Narrow ones,
+of a few pixels each, are test_gpu_backward_narrow.py's.)
 
 Tolerance, element by element: |difference| <= (2e-6 + 3e-7 n) times the sum
 of the terms' magnitudes.  The device recovers T in front of entry k by n - k
