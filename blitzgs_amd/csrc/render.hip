@@ -3487,10 +3487,14 @@ __device__ __forceinline__ int grad_slot(int lane)
 struct GradSum {
     float v;       // the term of accumulator slot grad_slot(lane)
     uint32_t cx;   // of this accumulator row
+    bool blended;  // FULL: a pixel blends the entry
 };
 
-// The sums of the four entries staged from j0 on.  grad_flush adds those whose
-// bit is set in `blended` to the accumulators.
+// The sums of the four entries staged from j0 on.  grad_flush adds the first
+// n of them to the accumulators; on the full-image path, where the forward marks
+// what it staged, those of them that a pixel blends, i.e. that have an alpha T
+// above zero (an entry that no pixel blends takes no sum: an image gradient that
+// is not finite would make its zero factors NaN).
 template <bool FULL, bool GEO>
 __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels<GEO>& g, const Stage& st,
                                              int j0, int lane)
@@ -3535,16 +3539,21 @@ __device__ __forceinline__ GradSum grad_sums(const float* rows, const GradPixels
     const float sum = grad_reduce<GEO>(swap32_add(gx, gy), p23, swap32_add(wxx, wxy), swap32_add(wyy, s),
                                        swap32_add(dot(g.dp[0]), dot(g.dp[1])), pab, pcd, pef, lane);
     lds_order();
-    return GradSum{grad_slot(lane) < 7 ? B.y * sum : sum, cx};   // slots 0 .. 6: the mean's and the conic's
+    bool blended = true;
+    if constexpr (FULL) {
+        const uint64_t b = gs::ballot((v.x + v.y) + (v.z + v.w) != 0.f);
+        blended = ((((uint32_t)b | (uint32_t)(b >> 32)) >> (2 * e)) & 0x03030303u) != 0;   // the entry's lanes
+    }
+    return GradSum{grad_slot(lane) < 7 ? B.y * sum : sum, cx, blended};   // slots 0 .. 6: the mean's and the conic's
 }
 
 template <bool FULL, bool GEO>
 __device__ __forceinline__ void grad_flush(const float* rows, const GradPixels<GEO>& g, const Stage& st,
-                                           int j0, uint32_t blended, int lane, float* __restrict__ gacc)
+                                           int j0, int n, int lane, float* __restrict__ gacc)
 {
     const GradSum t = grad_sums<FULL, GEO>(rows, g, st, j0, lane);
     const int i = grad_slot(lane);
-    const bool on = ((blended >> ((lane >> 1) & 3)) & 1u) != 0 && i < (GEO ? 16 : 11) && !(FULL && (i == 2 || i == 3));
+    const bool on = (FULL ? t.blended && i != 2 && i != 3 : ((lane >> 1) & 3) < n) && i < (GEO ? 16 : 11);
     if (on) unsafeAtomicAdd(gacc + (size_t)t.cx * 16 + i, t.v);
 }
 
@@ -3772,12 +3781,6 @@ __device__ __forceinline__ void render_bwd_body(
         }
         __syncthreads();
         for (int j0 = 0; j0 < cnt; j0 += GRAD_SLOTS) {
-            // the entries of this group that a pixel blends: on the split path
-            // every marked one; on the full-image path, where the forward marks
-            // what it staged, those found here (an entry that no pixel blends
-            // takes no sum: a gradient that is not finite would make its zero
-            // factors NaN)
-            uint32_t blended = FULL ? 0u : (1u << min(cnt - j0, GRAD_SLOTS)) - 1u;
 #pragma unroll
             for (int s = 0; s < GRAD_SLOTS; s++) {
                 const int j = j0 + s;
@@ -3785,7 +3788,6 @@ __device__ __forceinline__ void render_bwd_body(
                 const float4 B = st.b[j];
                 const float4 Cc = st.c[j];
                 const BwdEval e = bwd_eval(kc, A, B, Cc);
-                if constexpr (FULL) blended |= gs::ballot(e.valid) != 0 ? 1u << s : 0u;
                 float m_dp = 0.f;
                 if constexpr (GEO) {
                     m_dp = st_map[j] * dm[0];
@@ -3793,8 +3795,7 @@ __device__ __forceinline__ void render_bwd_body(
                 }
                 grad_put(rows, s, lane, bwd_apply<FULL, GEO>(px_st, kc, A, B, Cc, e, m_dp));
             }
-            if (FULL && blended == 0u) continue;
-            grad_flush<FULL, GEO>(rows, gp, st, j0, blended, lane, gacc);
+            grad_flush<FULL, GEO>(rows, gp, st, j0, cnt - j0, lane, gacc);
         }
         __syncthreads();
     }
