@@ -3390,9 +3390,9 @@ __device__ __forceinline__ BwdTerms bwd_apply(BwdPixel& p, const BwdConst& k, co
 // Measured
 // (render backward, per pixel -> with the moments; in brackets now, with the
 // offsets one by one and the marks): 6M aerial Gaussians at 1600x1066 642 ->
-// 510 us (437), 1M wide ones at 1920x1080 367 -> 284 us (267), the full-image
-// path's 2M at 1237x822 377 -> 225 us (235); render_geo's 6M 909 us (600), 1M
-// 565 us (350).  Tried: the sums as a contraction on the matrix
+// 510 us (439), 1M wide ones at 1920x1080 367 -> 284 us (263), the full-image
+// path's 2M at 1237x822 377 -> 225 us (227); render_geo's 6M 909 us (584), 1M
+// 565 us (339).  Tried: the sums as a contraction on the matrix
 // cores, v_mfma_f32_16x16x4_f32 with four entries' rows against per-pixel
 // constants (equal accuracy): 700 us at 6M, because a float32 MFMA and the
 // VALU do not overlap on this target (a loop of one MFMA and 16 FMAs takes 108
@@ -3656,8 +3656,9 @@ __device__ void bwd_schedule_block(unsigned x, unsigned gx, unsigned gy, unsigne
 // GEO: render_geo (reference _r backward.cu:393-405,427-432,476-490): the five
 // maps enter dL/dalpha beside the colour, and their gradients
 // alpha T dL/dmap go to accumulator slots 11..15.
-// Occupancy: six waves per SIMD (80 VGPRs, 6.3 KB of LDS) except with
-// render_geo's map terms.
+// Occupancy: six waves per SIMD (80 VGPRs, 6.3 KB of LDS); with render_geo's
+// map terms five (96 VGPRs, four values spilled; left to itself the compiler takes 102 and four
+// waves: 608 -> 584 us at 6M, 362 -> 339 us at 1M).
 template <bool FULL, bool GEO>
 __device__ __forceinline__ void render_bwd_body(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
@@ -3802,7 +3803,7 @@ __device__ __forceinline__ void render_bwd_body(
 }
 
 template <bool FULL, bool GEO = false>
-__global__ __launch_bounds__(64, GEO ? 4 : 6) void render_bwd_kernel(
+__global__ __launch_bounds__(64, GEO ? 5 : 6) void render_bwd_kernel(
     int W, int H, unsigned gx, unsigned gy, unsigned sgx, unsigned NS, const uint2* __restrict__ ranges,
     const uint32_t* __restrict__ clist, const float4* __restrict__ rec, const uint8_t* __restrict__ cl,
     const float* __restrict__ bg, const float* __restrict__ final_T, const uint32_t* __restrict__ n_contrib_px,
