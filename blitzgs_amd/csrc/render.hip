@@ -194,8 +194,8 @@ struct BinLayout {
     size_t sortkey, point_list, keys, clist, smask, total;
 };
 
-// The compact list comes first: it is the only array the blend, the backward
-// and the depth pass read.  The point list and its keys (written on request,
+// The compact list comes first: the blend and the depth pass read no other
+// array, the backward also the staged masks, which come last.  The point list and its keys (written on request,
 // after the forward) follow it, and the forward's unsorted keys use their
 // space as scratch.  Nothing at or past an offset depends on R except through
 // that offset, so a buffer laid out for a capacity C >= R serves R: its

